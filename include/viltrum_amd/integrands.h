@@ -147,6 +147,18 @@ typedef struct vmx_integrand {
 
 namespace vmx {
 
+/* Whether a math policy asks for parameters to be loaded ahead of their use, several rows at
+   a time (`loads_ahead`): where few waves run, a loop over rows is otherwise a chain of load
+   latencies; where the chip is full, the registers are better spent otherwise. */
+template <class M, class = void>
+struct LoadsAhead {
+    static constexpr bool value = false;
+};
+template <class M>
+struct LoadsAhead<M, decltype(void(M::loads_ahead))> {
+    static constexpr bool value = true;
+};
+
 /* `eval<M, D>` takes a math policy M with static exp, sin and cos overloads for float
    and double; host and device code each supply their own. */
 
@@ -220,6 +232,19 @@ struct Blobs {
         return q;
     }
 
+    template <class M, int D>
+    VMX_HD static T add_blob(T s, const T* b, const T* x) {
+        T dx, dy;
+        if constexpr (D == 3) {
+            dx = x[0] - M::fma(b[2], x[2], b[0]);
+            dy = x[1] - M::fma(b[3], x[2], b[1]);
+        } else {  // t = 0: the centre is (cx, cy)
+            dx = x[0] - b[0];
+            dy = x[1] - b[1];
+        }
+        return M::fma(b[6], M::exp(-M::fma(b[5], dy * dy, b[4] * (dx * dx))), s);
+    }
+
     /* Sums in blob order.  M::fma(a, b, c) is a*b + c under the policy's rounding; with
        the unfused policies every value is the plain expression
        s + w*exp(-(ax*(dx*dx) + ay*(dy*dy))), dx = x - (cx + vx*t). */
@@ -227,17 +252,18 @@ struct Blobs {
     VMX_HD T eval(const T* x) const {
         static_assert(D == 2 || D == 3, "blob family is 2-D or 3-D");
         T s = T(0);
-        for (int k = 0; k < nblobs; ++k) {
-            const T* b = blob[k];
-            T dx, dy;
-            if constexpr (D == 3) {
-                dx = x[0] - M::fma(b[2], x[2], b[0]);
-                dy = x[1] - M::fma(b[3], x[2], b[1]);
-            } else {  // t = 0: the centre is (cx, cy)
-                dx = x[0] - b[0];
-                dy = x[1] - b[1];
+        if constexpr (LoadsAhead<M>::value) {
+            constexpr int CH = 4;  // rows loaded together, past the last blob too (rows exist to VMX_MAX_BLOBS)
+            static_assert(VMX_MAX_BLOBS % CH == 0, "whole chunks of rows");
+            for (int k = 0; k < nblobs; k += CH) {
+                T b[CH][7];
+                for (int u = 0; u < CH; ++u)
+                    for (int i = 0; i < 7; ++i) b[u][i] = blob[k + u][i];
+                for (int u = 0; u < CH; ++u)
+                    if (k + u < nblobs) s = add_blob<M, D>(s, b[u], x);
             }
-            s = M::fma(b[6], M::exp(-M::fma(b[5], dy * dy, b[4] * (dx * dx))), s);
+        } else {
+            for (int k = 0; k < nblobs; ++k) s = add_blob<M, D>(s, blob[k], x);
         }
         if (wa != T(0)) s = s + wa * (M::sin(wfx * x[0]) * M::cos(wfy * x[1]));
         if (step_mode != 0) {

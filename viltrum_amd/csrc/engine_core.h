@@ -77,6 +77,8 @@ struct vmx_ctx {
     // busy rounds the last call of a workload class (and budget octave) needed: where the
     // round chunks shrink
     std::map<std::array<uint64_t, 7>, uint32_t> round_hint;
+    // workload classes whose jobs did not end inside k_grow: they run the round kernels
+    std::map<std::array<uint64_t, 7>, bool> grow_off;
     const Shape* trial = nullptr;
     std::vector<std::array<uint64_t, 6>> tuned_keys;
     // last result (for vmx_export_regions): gathered from device memory on demand
@@ -128,6 +130,16 @@ inline void* ensure(vmx_ctx::Buf& b, size_t bytes) {
         b.bytes = bytes;
     }
     return b.p;
+}
+
+/* No-alloc calls: the arenas are carved anew from the start of the fixed array. */
+inline void reset_fixed(vmx_ctx* ctx) {
+    for (vmx_ctx::Buf* b : {&ctx->tree, &ctx->regs, &ctx->lists, &ctx->misc, &ctx->bins2})
+        if (b->fixed) {
+            b->fixed->used = 0;
+            b->p = nullptr;
+            b->bytes = 0;
+        }
 }
 
 /* A batch whose (bin, footprint) pair total does not fit the 32-bit list offsets. */
@@ -262,10 +274,43 @@ void launch_expand(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int par, 
     vmx::k_expand_round<T, D, P, Math, false><<<blocks, vmx::GEN_THREADS, pre_bytes, st>>>(g, d_f, par);
 }
 
+/* Rough instruction count of one evaluation, for the choice of how regions are generated
+   (a user's functor: a middling guess). */
+template <typename P>
+double eval_work(const P&) {
+    return 100.0;
+}
 template <typename T>
-struct RocprimTemp {
-    size_t sort_bytes = 0, scan_bytes = 0;
-};
+double eval_work(const vmx::Poly<T>& p) {
+    return 30.0 + 12.0 * p.nterms;
+}
+template <typename T>
+double eval_work(const vmx::Blobs<T>& p) {  // FP64: the precise exp, sin and cos
+    return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 80.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
+}
+template <typename T, typename Inner, int DF, int RD>
+double eval_work(const vmx::Fubini<T, Inner, DF, RD>& p) {
+    return double(p.mc) * (80.0 + eval_work(p.in));
+}
+
+/* Whether k_grow is built for a pipeline: a child of a split in the registers of one lane
+   (D <= 3), with the learned priority the network beside it in LDS (D <= 2). */
+template <int D>
+constexpr bool grow_built(bool learn) {
+    return D <= (learn ? 2 : 3);
+}
+
+template <typename T, int D, typename P, typename Math>
+void launch_grow(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int32_t* leaf, int select, hipStream_t st) {
+    if constexpr (std::is_same<T, float>::value && grow_built<D>(true) && !vmx::IsFubini<P>::value) {
+        if (learn) {
+            vmx::k_grow<T, D, P, Math, true><<<g.J, vmx::GROW_THREADS, 0, st>>>(g, d_f, leaf, select);
+            return;
+        }
+    }
+    if constexpr (grow_built<D>(false))
+        vmx::k_grow<T, D, P, Math, false><<<g.J, vmx::GROW_THREADS, 0, st>>>(g, d_f, leaf, select);
+}
 
 /* One (scalar, D, family) batch through the device pipeline (pipeline.h). */
 template <typename T, int D, typename P, typename Math>

@@ -68,6 +68,9 @@ struct Layout {
 
 /* float -> bfloat16, round to nearest even (NaN stays a quiet NaN). */
 VMX_HD inline uint16_t f2bf(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(uint16_t, __bf16(x));  // v_cvt_pk_bf16_f32: one instruction for six
+#endif
     uint32_t u = __builtin_bit_cast(uint32_t, x);
     if ((u & 0x7fffffffu) > 0x7f800000u) return uint16_t((u >> 16) | 0x40u);
     u += 0x7fffu + ((u >> 16) & 1u);
@@ -77,12 +80,7 @@ VMX_HD inline float bf2f(uint16_t h) { return __builtin_bit_cast(float, uint32_t
 
 /* number of halvings along a dim, from the dyadic code (leading 1 then the path) */
 VMX_HD inline int code_depth(uint32_t code) {
-    int n = 0;
-    while (code > 1u) {
-        code >>= 1;
-        ++n;
-    }
-    return n;
+    return code > 1u ? 31 - __builtin_clz(code) : 0;
 }
 
 /* Features of one region, handed to put(i, value) for i = 0..KP-1 (floats before BF16

@@ -55,6 +55,12 @@ struct FastMath {
     __device__ static double cos2pi(double p) { return ::cos(6.283185307179586476925286766559 * p); }
 };
 
+/* A policy for region generation, whose launches leave most of the chip idle. */
+template <class M>
+struct Ahead : M {
+    static constexpr bool loads_ahead = true;
+};
+
 /* 16-bit histogram key of a non-negative error: its top 16 bits (order preserving). */
 __device__ inline uint32_t key16(float b) { return __float_as_uint(b) >> 16; }
 __device__ inline uint32_t key16(double b) { return uint32_t(uint64_t(__double_as_longlong(b)) >> 48); }

@@ -33,7 +33,7 @@ constexpr uint32_t NONE = 0xFFFFFFFFu;
 constexpr int MAX_JOBS = 4096;
 constexpr int GEN_THREADS = 256;
 
-enum : uint32_t { JF_CAPACITY = 1, JF_DEPTH = 2, JF_ROUNDS = 4, JF_EMPTY_BIN = 16, JF_LEAVES = 32 };
+enum : uint32_t { JF_CAPACITY = 1, JF_DEPTH = 2, JF_ROUNDS = 4, JF_EMPTY_BIN = 16, JF_LEAVES = 32, JF_HANDOVER = 64 };
 
 template <typename T>
 struct Job {
@@ -51,6 +51,7 @@ struct Job {
     int32_t lfloor;  // with learn: every dim is first halved lfloor times, widest first
     float lres[VMX_MAX_DIM];  // log2 of the bin count per dim (0 for integrated dims)
     uint32_t defer_m;  // deferred rounds: at most about this many expansions per round
+    uint32_t grow_stop;  // k_grow hands the job over to the round kernels at this pool size
 };
 
 struct JobRt {
@@ -205,6 +206,21 @@ struct TeamShape {
     static constexpr int TEAM = D <= 2 ? 8 : (D == 3 ? 32 : (D <= 5 ? 64 : 256));
 };
 
+/* Orders a team's LDS accesses.  A team of up to 64 lanes lies in one wave, whose LDS
+   operations execute in order: only the compiler has to keep them so, no barrier of the
+   block is needed (a round's step had about ten of them).  Every lane of the wave (of the
+   block for larger teams) calls it. */
+template <int TEAM>
+__device__ inline void team_sync() {
+    if constexpr (TEAM <= 64) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
 template <typename T, int D>
 struct TeamLds {
     static constexpr int K = pow3(D), KM = pow3(D - 1);
@@ -217,33 +233,100 @@ struct TeamLds {
     int32_t deep[2];  // children that qualify in the same round (slot, or -1)
 };
 
+/* Calls fn(c, d, full, below, jl, at) for every line (c, d, jl) of nc regions, shared
+   among a team's lanes: line jl along dim d has the nodes full, full + below and
+   full + 2 below (below = 3^d) and number at = (c * D + d) * 3^(D-1) + jl.  Up to D = 3 all
+   lines of all dims and both regions form one list (D = 2: 12 lines on 8 lanes), where a
+   loop per region and dim would leave most lanes idle (3 of 8 busy); above, a dim's lines
+   fill the team and the loops keep every 3^d a constant. */
+template <int D, int TEAM, typename Fn>
+__device__ inline void for_team_lines(int nc, int lane, Fn fn) {
+    constexpr int KM = pow3(D - 1);
+    if constexpr (D <= 3) {
+        for (int q = lane; q < nc * D * KM; q += TEAM) {
+            const int c = q / (D * KM), d = (q / KM) % D, jl = q % KM;
+            int full = 0, below = 1;
+#pragma unroll
+            for (int e = 0; e < D; ++e)
+                if (d == e) {
+                    full = (jl % pow3(e)) + (jl / pow3(e)) * pow3(e) * 3;
+                    below = pow3(e);
+                }
+            fn(c, d, full, below, jl, q);
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (c >= nc) break;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const int below = pow3(d);
+                for (int jl = lane; jl < KM; jl += TEAM)
+                    fn(c, d, (jl % below) + (jl / below) * below * 3, below, jl, (c * D + d) * KM + jl);
+            }
+        }
+    }
+}
+
+/* (err, dim) of a region with box [lo, hi] from its folded error along each dim, E[d *
+   stride], under the chosen heuristic. */
+template <typename T, int D>
+__device__ inline void heuristic_pick(const T* E, int stride, const T* lo, const T* hi, int heur, T& err_out,
+                                      int& dim_out) {
+    const T vol = box_volume<T, D>(lo, hi);
+    if (heur == 0) {
+        const double size_weight = 1.e-5, min_size = 1.e-37;
+        T max_err = vol * E[0];
+        const T ext0 = hi[0] - lo[0];
+        if (ext0 < min_size || visnan(ext0))
+            max_err = 0;
+        else
+            max_err += size_weight * vabs(ext0);
+        int max_dim = 0;
+#pragma unroll
+        for (int d = 1; d < D; ++d) {
+            const T ext = hi[d] - lo[d];
+            T err = vol * E[d * stride] + size_weight * vabs(ext);
+            if (ext < min_size) err = 0;
+            if (err >= max_err) {
+                max_err = err;
+                max_dim = d;
+            }
+        }
+        err_out = max_err;
+        dim_out = max_dim;
+    } else {
+        T max_err = 0;
+        int max_dim = 0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const T err = vol * E[d * stride];
+            if (err > max_err) {
+                max_err = err;
+                max_dim = d;
+            }
+        }
+        err_out = max_err;
+        dim_out = max_dim;
+    }
+}
+
 /* Line errors and folds for `nc` regions held in L.cv[c] with boxes L.box[c]; lanes
    `lane` of `team`; returns (err, dim) of region c in lane c (c < nc).  Every lane of
-   the block must call it (it contains __syncthreads). */
+   the team's wave (of the block for teams above 64 lanes) calls it. */
 template <typename T, int D, int TEAM>
 __device__ inline void team_heuristic(TeamLds<T, D>& L, int nc, int heur, int lane, bool active, T& err_out,
                                       int& dim_out) {
     constexpr int KM = pow3(D - 1);
-    // line (c, d, jl) of region c along dim d lands at (c * D + d) * KM + jl; the loops
-    // over c and d are unrolled so every 3^d below is a compile-time constant
-    if (active) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            if (c >= nc) break;
+    // line (c, d, jl) of region c along dim d lands at (c * D + d) * KM + jl
+    if (active)
+        for_team_lines<D, TEAM>(nc, lane, [&](int c, int, int full, int below, int, int at) {
             const T* v = L.cv[c];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int below = pow3(d);
-                for (int jl = lane; jl < KM; jl += TEAM) {
-                    const int full = (jl % below) + (jl / below) * below * 3;
-                    const T p0 = v[full], p1 = v[full + below], p2 = v[full + 2 * below];
-                    const T sm = simpson(p0, p1, p2), tz = trapezoid(p0, p2);
-                    L.e[0][(c * D + d) * KM + jl] = heur == 0 ? metric_relative(sm, tz) : metric_absolute(sm, tz);
-                }
-            }
-        }
-    }
-    __syncthreads();
+            const T p0 = v[full], p1 = v[full + below], p2 = v[full + 2 * below];
+            const T sm = simpson(p0, p1, p2), tz = trapezoid(p0, p2);
+            L.e[0][at] = heur == 0 ? metric_relative(sm, tz) : metric_absolute(sm, tz);
+        });
+    team_sync<TEAM>();
     int buf = 0;
 #pragma unroll
     for (int lev = 0; lev < D - 1; ++lev) {
@@ -255,47 +338,11 @@ __device__ inline void team_heuristic(TeamLds<T, D>& L, int nc, int heur, int la
                 L.e[buf ^ 1][g * KM + k] = simpson(in[3 * k], in[3 * k + 1], in[3 * k + 2]);
             }
         buf ^= 1;
-        __syncthreads();
+        team_sync<TEAM>();
     }
     if (active && lane < nc) {
         const int c = lane;
-        const T* lo = L.box[c][0];
-        const T* hi = L.box[c][1];
-        const T vol = box_volume<T, D>(lo, hi);
-        const T* E = L.e[buf] + c * D * KM;  // E[d * KM] = folded error of dim d
-        if (heur == 0) {
-            const double size_weight = 1.e-5, min_size = 1.e-37;
-            T max_err = vol * E[0];
-            const T ext0 = hi[0] - lo[0];
-            if (ext0 < min_size || visnan(ext0))
-                max_err = 0;
-            else
-                max_err += size_weight * vabs(ext0);
-            int max_dim = 0;
-            for (int d = 1; d < D; ++d) {
-                const T ext = hi[d] - lo[d];
-                T err = vol * E[d * KM] + size_weight * vabs(ext);
-                if (ext < min_size) err = 0;
-                if (err >= max_err) {
-                    max_err = err;
-                    max_dim = d;
-                }
-            }
-            err_out = max_err;
-            dim_out = max_dim;
-        } else {
-            T max_err = 0;
-            int max_dim = 0;
-            for (int d = 0; d < D; ++d) {
-                const T err = vol * E[d * KM];
-                if (err > max_err) {
-                    max_err = err;
-                    max_dim = d;
-                }
-            }
-            err_out = max_err;
-            dim_out = max_dim;
-        }
+        heuristic_pick<T, D>(L.e[buf] + c * D * KM, KM, L.box[c][0], L.box[c][1], heur, err_out, dim_out);
     }
 }
 
@@ -375,7 +422,7 @@ struct GenArgs {
     uint32_t* cstart;  // [2*J] first slot of the round's candidates (they are contiguous)
     uint32_t* ncand;   // [2*J] number of candidates
     T* theta;         // [J]
-    uint32_t* rounds; // rounds that had candidates
+    uint32_t* rounds; // [0] rounds that had candidates, [1] steps of k_grow
     uint32_t* depth;  // [D] most splits along each dim over all nodes (block maxima)
     uint32_t J;
     uint32_t max_rounds;
@@ -436,13 +483,14 @@ struct LearnLds {
    (lane 0..TEAM-1) and written as BF16 to rows[0..1]; jb == nullptr writes zero rows.
    The values are those of nn::region_features bit for bit: s is a max, and each fold
    adds its line terms in the same order.  Lane c < 2 gets child c's s and total
-   depth.  Every lane of the block calls it (it contains __syncthreads). */
+   depth.  Every lane of the team's wave calls it (learned priorities: teams of up to 64
+   lanes). */
 template <typename T, int D, int TEAM>
 __device__ inline void team_child_features(const TeamLds<T, D>& L, const Job<T>* jb, const uint32_t* pcode, int dim,
                                            int lane, uint16_t (*rows)[nn::Dims<D>::KP + 8], float* terms,
                                            float& s_lane, int& depth_lane) {
     constexpr int K = pow3(D), KM = pow3(D - 1), KP = nn::Dims<D>::KP;
-    __syncthreads();  // terms overwrite the heuristic's line errors
+    team_sync<TEAM>();  // terms overwrite the heuristic's line errors
     // s of both children: lane-strided maxima, then a butterfly inside the team's lanes
     float m0 = 0.f, m1 = 0.f;
     if (jb)
@@ -461,63 +509,138 @@ __device__ inline void team_child_features(const TeamLds<T, D>& L, const Job<T>*
         rows[c][3 * D + k] = jb ? nn::f2bf(float(L.cv[c][k]) * (c ? inv1 : inv0)) : uint16_t(0);
     }
     if (jb) {
-        // term (c, d, jl) at (c * D + d) * KM + jl; c and d unrolled (constant 3^d)
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int below = pow3(d);
-                for (int jl = lane; jl < KM; jl += TEAM) {
-                    const int full = (jl % below) + (jl / below) * below * 3;
-                    const float p0 = float(L.cv[c][full]), p1 = float(L.cv[c][full + below]),
-                                p2 = float(L.cv[c][full + 2 * below]);
-                    const float diff = vabs(simpson(p0, p1, p2) - trapezoid(p0, p2));
-                    float w = 1.f;
-                    int rr = jl;
-                    for (int e = 0; e < D - 1; ++e) {
-                        const int dg = rr % 3;
-                        rr /= 3;
-                        w *= (dg == 1) ? (4.f / 6.f) : (1.f / 6.f);
-                    }
-                    terms[(c * D + d) * KM + jl] = w * diff;
-                }
+        for_team_lines<D, TEAM>(2, lane, [&](int c, int, int full, int below, int jl, int at) {
+            const float p0 = float(L.cv[c][full]), p1 = float(L.cv[c][full + below]),
+                        p2 = float(L.cv[c][full + 2 * below]);
+            const float diff = vabs(simpson(p0, p1, p2) - trapezoid(p0, p2));
+            float w = 1.f;
+            int rr = jl;
+            for (int e = 0; e < D - 1; ++e) {
+                const int dg = rr % 3;
+                rr /= 3;
+                w *= (dg == 1) ? (4.f / 6.f) : (1.f / 6.f);
             }
+            terms[at] = w * diff;
+        });
     }
-    __syncthreads();
-    if (lane < 2 * D) {
+    team_sync<TEAM>();
+    int depth = 1;  // of either child: the parent's splits and one more
+#pragma unroll
+    for (int d = 0; d < D; ++d) depth += jb ? nn::code_depth(pcode[d]) : 0;
+    if (lane < 2 * D) {  // a child and dim per lane
         const int c = lane / D, d = lane % D;
-        float acc = 0.f;
-        if (jb)
-            for (int jl = 0; jl < KM; ++jl) acc += terms[(c * D + d) * KM + jl];
-        rows[c][3 * D + K + d] = jb ? nn::f2bf(acc * (c ? inv1 : inv0)) : uint16_t(0);
-    }
-    for (int q = lane; q < 2 * (KP - 4 * D - K - 1); q += TEAM) {
-        const int c = q / (KP - 4 * D - K - 1), i = 4 * D + K + 1 + q % (KP - 4 * D - K - 1);
-        rows[c][i] = 0;
-    }
-    s_lane = 0.f;
-    depth_lane = 0;
-    if (lane < 2) {
-        const int c = lane;
         uint16_t* row = rows[c];
+        uint32_t code = pcode[0];
+#pragma unroll
+        for (int e = 1; e < D; ++e)
+            if (d == e) code = pcode[e];
+        float acc = 0.f, ctr = 0.f, res = 0.f;
+        int n = 0;
         if (jb) {
-            int depth = 0;
-            for (int d = 0; d < D; ++d) {
-                const T ctr = T((T(0.5) * (L.box[c][0][d] + L.box[c][1][d]) - jb->lo[d]) / (jb->hi[d] - jb->lo[d]));
-                row[d] = nn::f2bf(float(ctr));
-                const uint32_t code = d == dim ? pcode[d] * 2u + uint32_t(c) : pcode[d];
-                const int n = nn::code_depth(code);
-                depth += n;
-                row[D + d] = nn::f2bf(-float(n) * (1.f / 16.f));
-                row[2 * D + d] = nn::f2bf((jb->lres[d] - float(n)) * (1.f / 16.f));
-            }
-            row[4 * D + K] = nn::f2bf(float(depth) * (1.f / 32.f));
-            s_lane = c ? m1 : m0;
-            depth_lane = depth;
-        } else {
-            for (int i = 0; i < 3 * D; ++i) row[i] = 0;
-            row[4 * D + K] = 0;
+            for (int jl = 0; jl < KM; ++jl) acc += terms[(c * D + d) * KM + jl];
+            ctr = float(T((T(0.5) * (L.box[c][0][d] + L.box[c][1][d]) - jb->lo[d]) / (jb->hi[d] - jb->lo[d])));
+            n = nn::code_depth(code) + (d == dim ? 1 : 0);
+            acc *= c ? inv1 : inv0;
+            res = (jb->lres[d] - float(n)) * (1.f / 16.f);
         }
+        row[d] = nn::f2bf(ctr);
+        row[D + d] = jb ? nn::f2bf(-float(n) * (1.f / 16.f)) : uint16_t(0);
+        row[2 * D + d] = nn::f2bf(res);
+        row[3 * D + K + d] = nn::f2bf(acc);
+        if (d == 0) row[4 * D + K] = jb ? nn::f2bf(float(depth) * (1.f / 32.f)) : uint16_t(0);
+    }
+    // the padding, two values per store (F is even)
+    static_assert((4 * D + K + 1) % 2 == 0, "the padding starts at a 4-byte boundary");
+    for (int q = lane; q < KP - 4 * D - K - 1; q += TEAM) {
+        constexpr int H = (KP - 4 * D - K - 1) / 2;
+        reinterpret_cast<uint32_t*>(&rows[q / (H > 0 ? H : 1)][4 * D + K + 1])[q % (H > 0 ? H : 1)] = 0;
+    }
+    s_lane = lane == 0 ? m0 : m1;
+    depth_lane = depth;
+}
+
+/* Node values of the two children of L's node (boxes L.pbox and L.box, values L.pv, split
+   along L.dim): the inherited planes and the new ones into L.cv and to v at slots s0 and
+   s0 + 1; then lane c < 2 gets child c's heuristic error and split dim.  go: the team has
+   a node.  Every lane of the team's wave (of the block above 64 lanes) calls it. */
+template <typename T, int D, typename F, typename M>
+__device__ inline void team_children(TeamLds<T, D>& L, T* __restrict__ v, const F* __restrict__ f, int heur, int lane,
+                                     bool go, size_t s0, T& e, int& dm) {
+    constexpr int K = pow3(D), KM = pow3(D - 1);
+    constexpr int TEAM = TeamShape<D>::TEAM;
+    team_sync<TEAM>();
+    if (go) {
+        const int dim = L.dim;
+        const int stride = pow3(dim);
+        for (int idx = lane; idx < K; idx += TEAM) {
+            const int jd = digit3(idx, dim);
+            if (jd == 1) continue;
+            const int base = idx - jd * stride;
+            L.cv[0][idx] = L.pv[jd == 0 ? base : base + stride];
+            L.cv[1][idx] = L.pv[jd == 0 ? base + stride : base + 2 * stride];
+        }
+        for (int q = lane; q < 2 * KM; q += TEAM) {
+            const int c = q / KM, jj = q % KM;
+            T x[D];
+            const int idx = split_new_node<T, D>(L.pbox[0], L.pbox[1], dim, c, jj, x);
+            L.cv[c][idx] = f->template eval<M, D>(x);
+        }
+    }
+    team_sync<TEAM>();
+    if (go)
+        for (int q = lane; q < 2 * K; q += TEAM) v[(s0 + q / K) * K + q % K] = L.cv[q / K][q % K];
+    team_heuristic<T, D, TEAM>(L, 2, heur, lane, go, e, dm);
+}
+
+/* The learned priority of child c, from the network's output y for it, and its split dim.
+   lp = log2 of the predicted energy.  Stored as 2^(lp/4): the same order, and the whole
+   span of lp (about -450 for regions of zeros .. +50) stays inside the FP32 range, so no
+   clamp ties distinct predictions.  A child is held below 2^(-1/8) of its parent's
+   predicted energy (2^(-1/32) of its stored priority; the root's is +inf): priorities
+   fall strictly along every path, so b is the node's own priority and a subtree the
+   network overrates cannot tie with its ancestor and grow round after round.  e and dm
+   hold the heuristic's error and dim, which stand where the output is NaN. */
+template <typename T, int D>
+__device__ inline void learned_score(float y, float mu, float sigma, float sc, int depth, T parent_err, int lfloor,
+                                     const uint32_t* pcode, int dim, int c, T& e, int& dm) {
+    const float lp = y * sigma + mu + 2.f * log2f(vmax(sc, 0x1p-100f)) - float(depth);
+    if (lp == lp) {
+        const float cap = log2f(float(parent_err)) - 0.03125f;
+        e = T(exp2f(vmin(vmax(vmin(0.25f * lp, cap), -126.f), 60.f)));
+    }
+    // size floor: a child still wider than 2^-lfloor along some dim goes before every
+    // network-ranked region (2^(126 - depth/4) > 2^60, falling along paths) and is split
+    // along its widest dim.  Large regions are rare in the training pairs, so the
+    // network's ranking of them is the least reliable.
+    int nmin = 1 << 30, dmin = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        const uint32_t code = d == dim ? pcode[d] * 2u + uint32_t(c) : pcode[d];
+        const int n = nn::code_depth(code);
+        if (n < nmin) {
+            nmin = n;
+            dmin = d;
+        }
+    }
+    if (nmin < lfloor) {
+        e = T(exp2f(126.f - 0.25f * float(depth)));
+        dm = dmin;
+    }
+}
+
+/* First two entries of a child's path suffix-minimum stack, from its error e and its
+   parent's entries. */
+template <typename T>
+__device__ inline void child_stack(T e, T bp, T b1p, T& nb, T& nb1) {
+    if (e < bp) {
+        nb = e;
+        nb1 = T(INFINITY);
+    } else if (e < b1p) {
+        nb = bp;
+        nb1 = e;
+    } else {
+        nb = bp;
+        nb1 = b1p;
     }
 }
 
@@ -527,7 +650,7 @@ template <typename T, int D, typename F, typename M, bool LEARN>
 __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs, TeamLds<T, D>& L, int par,
                                    const uint32_t* pre, uint64_t w, bool has, int32_t direct, bool may_deepen,
                                    LearnLds<D>* ll, int team, SlotLds<GEN_THREADS / TeamShape<D>::TEAM>& sl) {
-    constexpr int K = pow3(D), KM = pow3(D - 1);
+    constexpr int K = pow3(D);
     constexpr int TEAM = TeamShape<D>::TEAM;
     constexpr int TPB = GEN_THREADS / TEAM;
     const int lane = threadIdx.x % TEAM;
@@ -563,31 +686,36 @@ __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs
         }
     }
     __syncthreads();
-    // two child slots per expanding team: one atomic per run of teams of the same job
-    if (threadIdx.x == 0) {
-        for (int a = 0; a < TPB;) {
-            if (!sl.want[a]) {
-                sl.slot[a] = -1;
-                ++a;
-                continue;
+    // two child slots per expanding team, one atomic per job among the block's teams: lane
+    // a of the first wave stands for team a
+    if (threadIdx.x < 64) {
+        const int a = int(threadIdx.x);
+        const bool want = a < TPB && sl.want[a < TPB ? a : 0] != 0;
+        const uint32_t ja = want ? sl.job[a] : 0u;
+        int32_t mine = -1;
+        uint64_t act = __ballot(want);
+        while (act) {
+            const int leader = __ffsll((unsigned long long)act) - 1;
+            const uint32_t j = __shfl(ja, leader);
+            const bool same_job = want && ja == j;
+            const uint64_t same = __ballot(same_job);
+            const uint32_t slots_wanted = 2u * uint32_t(__popcll(same));
+            uint32_t base = NONE;
+            if (a == leader) {
+                const Job<T>& jb = g.jobs[j];
+                base = atomicAdd(&g.rt[j].count, slots_wanted);
+                if (base + slots_wanted <= jb.node_base + jb.node_cap) {
+                    atomicAdd(&g.ncand[(par ^ 1) * J + j], slots_wanted);
+                } else {
+                    atomicOr(&g.rt[j].flags, JF_CAPACITY);
+                    base = NONE;
+                }
             }
-            const uint32_t j = sl.job[a];
-            int b = a, cnt = 0;
-            for (; b < TPB && (!sl.want[b] || sl.job[b] == j); ++b) cnt += sl.want[b];
-            const Job<T>& jb = g.jobs[j];
-            const uint32_t base = atomicAdd(&g.rt[j].count, 2u * uint32_t(cnt));
-            const bool fits = base + 2u * uint32_t(cnt) <= jb.node_base + jb.node_cap;
-            if (fits)
-                atomicAdd(&g.ncand[(par ^ 1) * J + j], 2u * uint32_t(cnt));
-            else
-                atomicOr(&g.rt[j].flags, JF_CAPACITY);
-            int k = 0;
-            for (int c = a; c < b; ++c) {
-                sl.slot[c] = (sl.want[c] && fits) ? int32_t(base + 2u * uint32_t(k)) : -1;
-                k += sl.want[c];
-            }
-            a = b;
+            base = __shfl(base, leader);
+            if (same_job && base != NONE) mine = int32_t(base + 2u * uint32_t(__popcll(same & ((1ull << a) - 1ull))));
+            act &= ~same;
         }
+        if (a < TPB) sl.slot[a] = mine;
     }
     __syncthreads();
     if (lane == 0 && sl.want[team] && sl.slot[team] >= 0) {
@@ -607,38 +735,14 @@ __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs
         }
         split_boxes<T, D>(plo, phi, dim, L.box[0][0], L.box[0][1], L.box[1][0], L.box[1][1]);
     }
-    __syncthreads();
+    team_sync<TEAM>();
     const bool go = L.go != 0;
     if (go)
         for (int k = lane; k < K; k += TEAM) L.pv[k] = t.v[size_t(L.node) * K + k];
-    __syncthreads();
-    if (go) {
-        const int dim = L.dim;
-        const int stride = pow3(dim);
-        const F& f = fs[L.job];
-        for (int idx = lane; idx < K; idx += TEAM) {
-            const int jd = digit3(idx, dim);
-            if (jd == 1) continue;
-            const int base = idx - jd * stride;
-            L.cv[0][idx] = L.pv[jd == 0 ? base : base + stride];
-            L.cv[1][idx] = L.pv[jd == 0 ? base + stride : base + 2 * stride];
-        }
-        for (int q = lane; q < 2 * KM; q += TEAM) {
-            const int c = q / KM, jj = q % KM;
-            T x[D];
-            const int idx = split_new_node<T, D>(L.pbox[0], L.pbox[1], dim, c, jj, x);
-            L.cv[c][idx] = f.template eval<M, D>(x);
-        }
-    }
-    __syncthreads();
-    if (go) {
-        const size_t s0 = size_t(L.slot);
-        for (int q = lane; q < 2 * K; q += TEAM) t.v[(s0 + q / K) * K + q % K] = L.cv[q / K][q % K];
-    }
     const int heur = go ? g.jobs[L.job].heur : 0;
     T e = 0;
     int dm = 0;
-    team_heuristic<T, D, TEAM>(L, 2, heur, lane, go, e, dm);
+    team_children<T, D, F, M>(L, t.v, fs + (go ? L.job : 0), heur, lane, go, size_t(L.slot), e, dm);
     if constexpr (LEARN) {
         // learned priority of both children (lane c scores child c); the heuristic's
         // split dim is kept, and its error stands in where the network output is NaN
@@ -657,39 +761,9 @@ __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs
                                         &ll->xs[0][0], LearnLds<D>::R, ll->h0(), ll->h1(), ll->h0(), ll->y);
         else
             nn::forward_block<KP>(ll->net, &ll->xs[0][0], LearnLds<D>::R, ll->h0(), ll->h1(), ll->h0(), ll->y);
-        if (lrn && lane < 2) {
-            // lp = log2 of the predicted energy.  Stored as 2^(lp/4): the same order, and
-            // the whole span of lp (about -450 for regions of zeros .. +50) stays inside
-            // the FP32 range, so no clamp ties distinct predictions.  A child is held
-            // below 2^(-1/8) of its parent's predicted energy (2^(-1/32) of its stored
-            // priority; the root's is +inf): priorities fall strictly along every path,
-            // so b is the node's own priority and a subtree the network overrates cannot
-            // tie with its ancestor and grow round after round.
-            const float lp = ll->y[team * 2 + lane] * ll->net.sigma + ll->net.mu +
-                             2.f * log2f(vmax(fsc, 0x1p-100f)) - float(fdepth);
-            if (lp == lp) {
-                const float cap = log2f(float(t.err[L.node])) - 0.03125f;
-                e = T(exp2f(vmin(vmax(vmin(0.25f * lp, cap), -126.f), 60.f)));
-            }
-            // size floor: a child still wider than 2^-lfloor along some dim goes before
-            // every network-ranked region (2^(126 - depth/4) > 2^60, falling along
-            // paths) and is split along its widest dim.  Large regions are rare in the
-            // training pairs, so the network's ranking of them is the least reliable.
-            const Job<T>& jb = g.jobs[L.job];
-            int nmin = 1 << 30, dmin = 0;
-            for (int d = 0; d < D; ++d) {
-                const uint32_t code = d == L.dim ? pcode[d] * 2u + uint32_t(lane) : pcode[d];
-                const int n = nn::code_depth(code);
-                if (n < nmin) {
-                    nmin = n;
-                    dmin = d;
-                }
-            }
-            if (nmin < jb.lfloor) {
-                e = T(exp2f(126.f - 0.25f * float(fdepth)));
-                dm = dmin;
-            }
-        }
+        if (lrn && lane < 2)
+            learned_score<T, D>(ll->y[team * 2 + lane], ll->net.mu, ll->net.sigma, fsc, fdepth, t.err[L.node],
+                                g.jobs[L.job].lfloor, pcode, L.dim, lane, e, dm);
     }
     if (go && lane < 2) {
         const int c = lane;
@@ -708,17 +782,8 @@ __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs
         t.err[s] = e;
         t.dim[s] = dm;
         const T bp = t.b[node], b1p = t.b1[node];
-        T nb, nb1;  // first two entries of the path's suffix-minimum stack
-        if (e < bp) {
-            nb = e;
-            nb1 = T(INFINITY);
-        } else if (e < b1p) {
-            nb = bp;
-            nb1 = e;
-        } else {
-            nb = bp;
-            nb1 = b1p;
-        }
+        T nb, nb1;
+        child_stack(e, bp, b1p, nb, nb1);
         t.b[s] = nb;
         t.b1[s] = nb1;
         L.deep[c] = may_deepen && nb >= g.theta[j] ? int32_t(s) : -1;
@@ -2232,5 +2297,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
 }  // namespace vmx
 
 #include "bins_rm.h"
+#include "grow.h"
 
 #endif

@@ -53,13 +53,35 @@ VMX_HD inline T node_coord(double p, T lo, T hi) {
     return T(p * (hi - lo) + lo);
 }
 
+/* x / 6.0, correctly rounded, for |x| in [2^-960, 2^1020], zero, infinite or NaN: the
+   product with RN(1/6), corrected by its exact remainder (division by a constant with a
+   fused multiply-add, Brisebarre, Muller and Raina 2004).  Four FP64 operations for the
+   dozen of the general quotient, which was most of a split's instructions. */
+VMX_HD inline double div6(double x) {
+    const double r = 1.0 / 6.0;
+    const double q = x * r;
+    const double e = __builtin_fma(-6.0, q, x);
+    return __builtin_fabs(e) > 0.0 ? __builtin_fma(e, r, q) : q;  // exact, zero, infinite or NaN: q
+}
+
 template <typename T>
 VMX_HD inline T simpson(T p0, T p1, T p2) {
     return T((p0 + 4.0 * p1 + p2) / 6.0);
 }
+/* of floats: the sum lies in div6's range, and 4 p1 is exact, so fusing it into the first
+   sum rounds as the two operations do */
+template <>
+VMX_HD inline float simpson<float>(float p0, float p1, float p2) {
+    return float(div6(__builtin_fma(4.0, double(p1), double(p0)) + double(p2)));
+}
+template <>
+VMX_HD inline double simpson<double>(double p0, double p1, double p2) {
+    const double x = p0 + 4.0 * p1 + p2, a = __builtin_fabs(x);
+    return (a >= 0x1p-960 && a <= 0x1p1000) || x == 0.0 ? div6(x) : x / 6.0;
+}
 template <typename T>
 VMX_HD inline T trapezoid(T p0, T p2) {
-    return T((p0 + p2) / 2.0);
+    return (p0 + p2) * T(0.5);  // T((p0 + p2) / 2.0): halving rounds the same in both types
 }
 template <typename T>
 VMX_HD inline T simpson_at(T t, T p0, T p1, T p2) {
@@ -91,7 +113,11 @@ VMX_HD inline T simpson_subrange_mul(T a, T b, T p0, T p1, T p2) {
 template <typename T>
 VMX_HD inline T metric_relative(T a, T b) {  // error_metric_relative(1e-37)
     const T ma = vmax(vabs(a), vabs(b));
-    if (double(ma) < 1.e-37) return vabs(b - a);
+    if constexpr (sizeof(T) == 4) {
+        if (ma <= 0x1.1039d4p-123f) return vabs(b - a);  // the largest float below 1e-37
+    } else {
+        if (double(ma) < 1.e-37) return vabs(b - a);
+    }
     return vabs(b - a) / ma;
 }
 template <typename T>

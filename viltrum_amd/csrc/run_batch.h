@@ -161,6 +161,36 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     std::array<uint64_t, 7> hint_key{};
     std::copy(tune_key.begin(), tune_key.end(), hint_key.begin());
     hint_key[6] = uint64_t(ilog2(n_max));
+    // One workgroup per integral generates it (grow.h) where that beats the rounds; both
+    // sides as measured (us).  k_grow: 8 steps while the tree is small, then a step for each
+    // 256 splits, issue-bound on one CU (5.5 and the 3^(D-1) evaluations of a lane; 14 for 3
+    // dims, 13 with the network), and the selection.  Rounds: about log2 N + 7 of two
+    // launches each, 20 and an evaluation (30 with the network), 2.5 ns a split, and the
+    // selection's launches.  One 2-D integral of 1024 / 2048 / 4096 regions: 370 / 400 / 500
+    // by rounds, 80 / 115 / 230 here; 64 learned ones of 4096 regions 1520 -> 430; 3 dims
+    // with 8 blobs cross over near 3000 regions, 2 dims with 64 blobs near 6000.  A larger
+    // integral alone starts here (the rounds of a handful of regions are all launch) and
+    // hands over once its pool fills the chip's first workgroups.  The reference's order
+    // replays a heap over the rounds' nodes.  VMX_DEFER chooses among forms of the rounds,
+    // so every call with it set runs them.
+    bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !std::getenv("VMX_DEFER");
+    bool grow_start = grow_all && J == 1;
+    if (grow_all) {
+        double grow_us = 0, rounds_us = 0, splits = 0;
+        for (uint32_t j = 0; j < J; ++j) {
+            const double eval_us = 0.0033 * eval_work(fparams[j]);  // 8 cycles an instruction
+            const double n = jobs[j].N, step_us = (learn ? 13.0 : (D <= 2 ? 5.5 : 14.0)) + 1.3 * vmx::pow3(D - 1) * eval_us;
+            grow_us = std::max(grow_us, 8.0 * (4.0 + eval_us) + (n / 256.0 + 4.0) * step_us + 10.0 + n / 100.0);
+            rounds_us = std::max(rounds_us, ((learn ? 30.0 : 20.0) + eval_us) * (7.0 + std::log2(n)) + 45.0);
+            splits += n;
+            grow_all &= n <= 6144;
+            grow_start &= n >= 256 && eval_us < (D <= 2 ? 10.0 : 2.0);
+        }
+        grow_all &= grow_us * double((J + 255) / 256) <= rounds_us + 0.0025 * splits;
+        grow_all &= order == VMX_ORDER_CANONICAL && !ctx->grow_off.count(hint_key);
+        for (auto& jb : jobs) jb.grow_stop = grow_all ? vmx::NONE : (D <= 2 ? 512u : 256u);
+    }
+    const bool grow = grow_all || grow_start;
     uint32_t max_depth[VMX_MAX_DIM] = {};
     uint64_t cap_mult = 8;
     if (const auto h = ctx->cap_hint.find(tune_key); h != ctx->cap_hint.end()) cap_mult = h->second;
@@ -303,8 +333,6 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             HIP_CHECK(hipStreamSynchronize(st));
             break;
         }
-        vmx::k_roots<T, D, P, Math><<<J, 256, 0, st>>>(d_jobs, d_rt, d_f, t, d_hist16, d_cstart, d_ncand);
-        HIP_CHECK(hipGetLastError());
         vmx::GenArgs<T> g{};
         g.jobs = d_jobs;
         g.rt = d_rt;
@@ -326,6 +354,17 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         g.nexp = d_nexp;
         g.exp = d_exp;
         g.chist = d_chist;
+        int32_t* grow_leaf = nullptr;
+        if (grow_all) {
+            ensure(ctx->regs, sizeof(int32_t) * n_reg);
+            grow_leaf = static_cast<int32_t*>(ctx->regs.p);
+        }
+        if (grow)
+            launch_grow<T, D, P, Math>(learn, g, d_f, grow_leaf, grow_all ? 1 : 0, st);
+        else
+            vmx::k_roots<T, D, P, Math><<<J, 256, 0, st>>>(d_jobs, d_rt, d_f, t, d_hist16, d_cstart, d_ncand);
+        HIP_CHECK(hipGetLastError());
+        if (grow_all) break;  // the regions' slots follow; the job states come back with the totals
         // rounds in chunks of round_chunk (even, so each chunk starts at parity 0); after
         // each chunk the candidate counts, job states and round counter are copied to
         // pinned memory.  The host checks chunk k while chunk k+1 runs, so the device is
@@ -414,7 +453,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         std::memcpy(rt.data(), slot(k) + sizeof(uint32_t) * 2 * J, sizeof(vmx::JobRt) * J);
         uint32_t small_h[16];
         std::memcpy(small_h, slot(k) + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, 64);
-        rounds = small_h[0];
+        rounds = small_h[0] + small_h[1];
         for (int d = 0; d < D; ++d) max_depth[d] = small_h[8 + d];
         bool cap_fail = false, too_deep = false;
         for (const auto& r : rt) {
@@ -429,7 +468,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             continue;
         }
         ctx->cap_hint[tune_key] = cap_mult;
-        ctx->round_hint[hint_key] = rounds;
+        ctx->round_hint[hint_key] = small_h[0];
         break;
     }
     const double ms_gen = ms_since(t_start);
@@ -484,103 +523,106 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     }
     const bool one_sort = key_bits64 <= 64;
     size_t sort_bytes = 0, sort64_bytes = 0;
-    HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                                  (int32_t*)nullptr, (int32_t*)nullptr, size_t(n_reg), 0, 32, st)));
-    HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(nullptr, sort64_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
-                                                  (int32_t*)nullptr, (int32_t*)nullptr, size_t(n_reg), 0,
-                                                  std::max(1, std::min(64, key_bits64)), st)));
-    sort_bytes = std::max(sort_bytes, sort64_bytes);
-    Measure ms;
-    ms.take<int32_t>(cap_total);   // bucket
-    ms.take<uint8_t>(cap_total);   // bstate
-    ms.take<int32_t>(n_reg);       // leaf slots
-    ms.take<int32_t>(n_reg);       // sort values tmp
-    ms.take<uint64_t>(n_reg);      // sort keys
-    ms.take<uint64_t>(n_reg);      // sort keys tmp
-    ms.take<char>(sort_bytes + 256);
-    ensure(ctx->regs, ms.used);
-    Carve cs(ctx->regs);
-    int32_t* d_bucket = cs.take<int32_t>(cap_total);
-    uint8_t* d_bstate = cs.take<uint8_t>(cap_total);
-    int32_t* d_leaf = cs.take<int32_t>(n_reg);
-    int32_t* d_leaf_tmp = cs.take<int32_t>(n_reg);
-    uint64_t* d_keys64 = cs.take<uint64_t>(n_reg);
-    uint64_t* d_keys64_tmp = cs.take<uint64_t>(n_reg);
-    uint32_t* d_keys = reinterpret_cast<uint32_t*>(d_keys64);
-    uint32_t* d_keys_tmp = reinterpret_cast<uint32_t*>(d_keys64_tmp);
-    void* d_sort_tmp = cs.take<char>(sort_bytes + 256);
-    const unsigned cap_blocks = (cap_total + 255) / 256;
+    int32_t* d_leaf = static_cast<int32_t*>(ctx->regs.p);  // with grow_all: k_grow has filled it
     const unsigned reg_blocks = unsigned((n_reg + 255) / 256);
-    if (replay) {
-        std::vector<int32_t> all_leaves(n_reg);
-        for (uint32_t j = 0; j < J; ++j)
-            for (uint32_t i = 0; i < jobs[j].N; ++i) all_leaves[jobs[j].reg_base + i] = int32_t(jobs[j].node_base + i);
-        HIP_CHECK(hipMemcpyAsync(d_leaf, all_leaves.data(), sizeof(int32_t) * n_reg, hipMemcpyHostToDevice, st));
-        HIP_CHECK(hipStreamSynchronize(st));
-    } else if (order == VMX_ORDER_CANONICAL) {
-        vmx::k_sel_bound<T><<<J, 256, 0, st>>>(d_jobs, d_rt, d_hist16, d_leaf);
-        vmx::k_sel_gather<T><<<cap_blocks, 256, 0, st>>>(d_jobs, d_rt, t, cap_total, d_bucket);
-        vmx::k_sel_resolve<T, D><<<J, 256, 0, st>>>(d_jobs, d_rt, t, d_bucket, d_bstate);
-        vmx::k_leaves<T><<<cap_blocks, 256, 0, st>>>(d_jobs, d_rt, t, cap_total, d_leaf);
-        HIP_CHECK(hipGetLastError());
-        int32_t* vin = d_leaf;
-        int32_t* vout = d_leaf_tmp;
-        if (one_sort) {
-            vmx::k_leaf_keys64<D><<<reg_blocks, 256, 0, st>>>(d_leaf, t.code, t.job, uint32_t(n_reg), widths, d_keys64,
-                                                              d_leaf_tmp);
-            size_t bytes = sort_bytes;
-            HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(d_sort_tmp, bytes, d_keys64, d_keys64_tmp, d_leaf_tmp, d_leaf,
-                                                          size_t(n_reg), 0, std::max(1, key_bits64), st)));
-        } else {
-            // LSD passes: code_{D-1} ... code_0, then job
-            for (int which = D - 1; which >= (J > 1 ? -1 : 0); --which) {
-                vmx::k_leaf_keys<D><<<reg_blocks, 256, 0, st>>>(vin, t.code, t.job, uint32_t(n_reg), which, d_keys);
-                size_t bytes = sort_bytes;
-                HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(d_sort_tmp, bytes, d_keys, d_keys_tmp, vin, vout,
-                                                              size_t(n_reg), 0, 32, st)));
-                std::swap(vin, vout);
-            }
-        }
-        if (vin != d_leaf)
-            HIP_CHECK(hipMemcpyAsync(d_leaf, vin, sizeof(int32_t) * n_reg, hipMemcpyDeviceToDevice, st));
-        // a job with fewer than N leaves leaves -1 slots behind: k_prepare2 turns them into
-        // empty regions and the host rejects the result at its next synchronisation
-    } else {
-        // the reference's heap-array order: replay push_heap / pop_heap on the errors
-        std::vector<int32_t> all_leaves(n_reg);
-        for (uint32_t j = 0; j < J; ++j) {
-            const auto& jb = jobs[j];
-            const uint32_t cnt = rt[j].count - jb.node_base;
-            std::vector<T> err(cnt);
-            std::vector<int32_t> child(cnt);
-            HIP_CHECK(hipMemcpyAsync(err.data(), t.err + jb.node_base, sizeof(T) * cnt, hipMemcpyDeviceToHost, st));
-            HIP_CHECK(hipMemcpyAsync(child.data(), t.child + jb.node_base, sizeof(int32_t) * cnt,
-                                     hipMemcpyDeviceToHost, st));
+    if (!grow_all) {
+        HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr,
+                                                      (int32_t*)nullptr, (int32_t*)nullptr, size_t(n_reg), 0, 32, st)));
+        HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(nullptr, sort64_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
+                                                      (int32_t*)nullptr, (int32_t*)nullptr, size_t(n_reg), 0,
+                                                      std::max(1, std::min(64, key_bits64)), st)));
+        sort_bytes = std::max(sort_bytes, sort64_bytes);
+        Measure ms;
+        ms.take<int32_t>(cap_total);   // bucket
+        ms.take<uint8_t>(cap_total);   // bstate
+        ms.take<int32_t>(n_reg);       // leaf slots
+        ms.take<int32_t>(n_reg);       // sort values tmp
+        ms.take<uint64_t>(n_reg);      // sort keys
+        ms.take<uint64_t>(n_reg);      // sort keys tmp
+        ms.take<char>(sort_bytes + 256);
+        ensure(ctx->regs, ms.used);
+        Carve cs(ctx->regs);
+        int32_t* d_bucket = cs.take<int32_t>(cap_total);
+        uint8_t* d_bstate = cs.take<uint8_t>(cap_total);
+        d_leaf = cs.take<int32_t>(n_reg);
+        int32_t* d_leaf_tmp = cs.take<int32_t>(n_reg);
+        uint64_t* d_keys64 = cs.take<uint64_t>(n_reg);
+        uint64_t* d_keys64_tmp = cs.take<uint64_t>(n_reg);
+        uint32_t* d_keys = reinterpret_cast<uint32_t*>(d_keys64);
+        uint32_t* d_keys_tmp = reinterpret_cast<uint32_t*>(d_keys64_tmp);
+        void* d_sort_tmp = cs.take<char>(sort_bytes + 256);
+        const unsigned cap_blocks = (cap_total + 255) / 256;
+        if (replay) {
+            std::vector<int32_t> all_leaves(n_reg);
+            for (uint32_t j = 0; j < J; ++j)
+                for (uint32_t i = 0; i < jobs[j].N; ++i) all_leaves[jobs[j].reg_base + i] = int32_t(jobs[j].node_base + i);
+            HIP_CHECK(hipMemcpyAsync(d_leaf, all_leaves.data(), sizeof(int32_t) * n_reg, hipMemcpyHostToDevice, st));
             HIP_CHECK(hipStreamSynchronize(st));
-            struct E {
-                T err;
-                int32_t node;
-            };
-            auto cmp = [](const E& a, const E& b) { return a.err < b.err; };
-            std::vector<E> heap;
-            heap.reserve(jb.N + 1);
-            heap.push_back({err[0], 0});
-            for (uint32_t i = 0; i + 1 < jb.N; ++i) {
-                const E top = heap.front();
-                const int32_t ch = child[top.node];
-                if (ch < 0) throw VmxError(VMX_ERR_CAPACITY, "heap replay reached an unexpanded node");
-                const int32_t cl = ch - int32_t(jb.node_base);
-                std::pop_heap(heap.begin(), heap.end(), cmp);
-                heap.pop_back();
-                heap.push_back({err[cl], cl});
-                std::push_heap(heap.begin(), heap.end(), cmp);
-                heap.push_back({err[cl + 1], cl + 1});
-                std::push_heap(heap.begin(), heap.end(), cmp);
+        } else if (order == VMX_ORDER_CANONICAL) {
+            vmx::k_sel_bound<T><<<J, 256, 0, st>>>(d_jobs, d_rt, d_hist16, d_leaf);
+            vmx::k_sel_gather<T><<<cap_blocks, 256, 0, st>>>(d_jobs, d_rt, t, cap_total, d_bucket);
+            vmx::k_sel_resolve<T, D><<<J, 256, 0, st>>>(d_jobs, d_rt, t, d_bucket, d_bstate);
+            vmx::k_leaves<T><<<cap_blocks, 256, 0, st>>>(d_jobs, d_rt, t, cap_total, d_leaf);
+            HIP_CHECK(hipGetLastError());
+            int32_t* vin = d_leaf;
+            int32_t* vout = d_leaf_tmp;
+            if (one_sort) {
+                vmx::k_leaf_keys64<D><<<reg_blocks, 256, 0, st>>>(d_leaf, t.code, t.job, uint32_t(n_reg), widths, d_keys64,
+                                                                  d_leaf_tmp);
+                size_t bytes = sort_bytes;
+                HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(d_sort_tmp, bytes, d_keys64, d_keys64_tmp, d_leaf_tmp, d_leaf,
+                                                              size_t(n_reg), 0, std::max(1, key_bits64), st)));
+            } else {
+                // LSD passes: code_{D-1} ... code_0, then job
+                for (int which = D - 1; which >= (J > 1 ? -1 : 0); --which) {
+                    vmx::k_leaf_keys<D><<<reg_blocks, 256, 0, st>>>(vin, t.code, t.job, uint32_t(n_reg), which, d_keys);
+                    size_t bytes = sort_bytes;
+                    HIP_CHECK(hipError_t(rocprim::radix_sort_pairs(d_sort_tmp, bytes, d_keys, d_keys_tmp, vin, vout,
+                                                                  size_t(n_reg), 0, 32, st)));
+                    std::swap(vin, vout);
+                }
             }
-            for (uint32_t i = 0; i < jb.N; ++i) all_leaves[jb.reg_base + i] = int32_t(jb.node_base) + heap[i].node;
+            if (vin != d_leaf)
+                HIP_CHECK(hipMemcpyAsync(d_leaf, vin, sizeof(int32_t) * n_reg, hipMemcpyDeviceToDevice, st));
+            // a job with fewer than N leaves leaves -1 slots behind: k_prepare2 turns them into
+            // empty regions and the host rejects the result at its next synchronisation
+        } else {
+            // the reference's heap-array order: replay push_heap / pop_heap on the errors
+            std::vector<int32_t> all_leaves(n_reg);
+            for (uint32_t j = 0; j < J; ++j) {
+                const auto& jb = jobs[j];
+                const uint32_t cnt = rt[j].count - jb.node_base;
+                std::vector<T> err(cnt);
+                std::vector<int32_t> child(cnt);
+                HIP_CHECK(hipMemcpyAsync(err.data(), t.err + jb.node_base, sizeof(T) * cnt, hipMemcpyDeviceToHost, st));
+                HIP_CHECK(hipMemcpyAsync(child.data(), t.child + jb.node_base, sizeof(int32_t) * cnt,
+                                         hipMemcpyDeviceToHost, st));
+                HIP_CHECK(hipStreamSynchronize(st));
+                struct E {
+                    T err;
+                    int32_t node;
+                };
+                auto cmp = [](const E& a, const E& b) { return a.err < b.err; };
+                std::vector<E> heap;
+                heap.reserve(jb.N + 1);
+                heap.push_back({err[0], 0});
+                for (uint32_t i = 0; i + 1 < jb.N; ++i) {
+                    const E top = heap.front();
+                    const int32_t ch = child[top.node];
+                    if (ch < 0) throw VmxError(VMX_ERR_CAPACITY, "heap replay reached an unexpanded node");
+                    const int32_t cl = ch - int32_t(jb.node_base);
+                    std::pop_heap(heap.begin(), heap.end(), cmp);
+                    heap.pop_back();
+                    heap.push_back({err[cl], cl});
+                    std::push_heap(heap.begin(), heap.end(), cmp);
+                    heap.push_back({err[cl + 1], cl + 1});
+                    std::push_heap(heap.begin(), heap.end(), cmp);
+                }
+                for (uint32_t i = 0; i < jb.N; ++i) all_leaves[jb.reg_base + i] = int32_t(jb.node_base) + heap[i].node;
+            }
+            HIP_CHECK(hipMemcpyAsync(d_leaf, all_leaves.data(), sizeof(int32_t) * n_reg, hipMemcpyHostToDevice, st));
+            HIP_CHECK(hipStreamSynchronize(st));
         }
-        HIP_CHECK(hipMemcpyAsync(d_leaf, all_leaves.data(), sizeof(int32_t) * n_reg, hipMemcpyHostToDevice, st));
-        HIP_CHECK(hipStreamSynchronize(st));
     }
     const double ms_sel = ms_since(t_sel);
 
@@ -685,6 +727,29 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         pairs = w[2];
         nfp = w[3];
         std::memcpy(rt.data(), pin + sizeof(uint32_t) * 2 * J, sizeof(vmx::JobRt) * J);
+        if (grow_all) {
+            std::memcpy(w, pin + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, 2 * sizeof(uint32_t));
+            rounds = w[1];
+        }
+    }
+    if (grow_all) {
+        bool cap_fail = false, handed = false;
+        for (const auto& r : rt) {
+            if (r.flags & vmx::JF_DEPTH) throw VmxError(VMX_ERR_CAPACITY, "region tree deeper than 31 splits in one dim");
+            cap_fail |= (r.flags & vmx::JF_CAPACITY) != 0;
+            handed |= (r.flags & vmx::JF_HANDOVER) != 0;
+        }
+        if (cap_fail || handed) {
+            // once more, with more room or in the round kernels; nothing is in flight
+            if (cap_fail) {
+                if (cap_mult >= 64) throw VmxError(VMX_ERR_CAPACITY, "node capacity exceeded");
+                ctx->cap_hint[tune_key] = 2 * cap_mult;
+            } else {
+                ctx->grow_off[hint_key] = true;
+            }
+            if (ctx->noalloc) reset_fixed(ctx);
+            return run_batch<T, D, P, Math>(ctx, in, st, pairs_req);
+        }
     }
     check_pair_total(pairs64);
     if (order == VMX_ORDER_CANONICAL && !replay)
