@@ -1592,39 +1592,14 @@ __global__ void __launch_bounds__(64 * prep_wpb<D>())
     }
 }
 
-/* The merged FP64 marginal of a footprint's regions [i, e): sum of vol_r * marginal_r
-   in region order, MB = 3^db entries held in registers. */
-template <typename T, int MB>
-__device__ inline void merge_marginals(const RegionArrays<T>& r, const FootArrays<T>& f, uint32_t i, uint32_t e,
-                                       uint32_t id) {
-    double acc[MB];
-#pragma unroll
-    for (int k = 0; k < MB; ++k) acc[k] = 0.0;
-    for (uint32_t q = i; q < e; ++q) {
-        const double vol = double(r.vol[q]);
-#pragma unroll
-        for (int k = 0; k < MB; ++k) acc[k] += vol * r.marg[size_t(q) * MB + k];
-    }
-#pragma unroll
-    for (int k = 0; k < MB; ++k) f.marg[size_t(id) * MB + k] = acc[k];
-}
-
-/* One thread per footprint: bin-dim box, pixel box, and merged FP64 marginal
-   (sum of vol_r * marginal_r over its regions, in region order) or, unmerged, the
-   single region's (vol, marginal) so per-region sums keep the reference's rounding. */
+/* Bin-dim box and pixel box of a footprint whose regions are [i, e). */
 template <typename T, int D>
-__global__ void k_footprints(const Job<T>* __restrict__ jobs, RegionArrays<T> r, FootArrays<T> f, uint32_t n,
-                             int mb, int merge) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !r.fpflag[i]) return;
-    const uint32_t id = r.fpid[i];
-    uint32_t e = i + 1;
-    while (e < n && !r.fpflag[e]) ++e;
-    const uint32_t j = r.job[i];
-    const Job<T>& jb = jobs[j];
+__device__ inline void footprint_boxes(const Job<T>& jb, const RegionArrays<T>& r, const FootArrays<T>& f, uint32_t i,
+                                       uint32_t e, uint32_t id, uint32_t j) {
     f.first[id] = i;
     f.count[id] = e - i;
     f.job[id] = j;
+    uint32_t np = 1;
     for (int d = 0; d < 3; ++d) {
         uint64_t a = 0, z = 1;
         if (d < jb.db) {
@@ -1635,23 +1610,83 @@ __global__ void k_footprints(const Job<T>* __restrict__ jobs, RegionArrays<T> r,
         }
         f.box[size_t(id) * 6 + 2 * d] = uint32_t(a);
         f.box[size_t(id) * 6 + 2 * d + 1] = uint32_t(z);
+        np *= uint32_t(z) - uint32_t(a);
     }
-    {
-        const uint32_t* bx = f.box + size_t(id) * 6;
-        f.npairs[id] = (bx[1] - bx[0]) * (bx[3] - bx[2]) * (bx[5] - bx[4]);
+    f.npairs[id] = np;
+}
+
+/* One thread per region that starts a footprint, where regions do not merge (no merging
+   asked for, or every dim has bins): its boxes, and its (vol, marginal) apart, so
+   per-region sums keep the reference's rounding; a merging batch multiplies them. */
+template <typename T, int D>
+__global__ void k_footprints1(const Job<T>* __restrict__ jobs, RegionArrays<T> r, FootArrays<T> f, uint32_t n,
+                              int mb, int merge) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t j = r.job[i];
+    const Job<T>& jb = jobs[j];
+    const uint32_t id = r.fpid[i];
+    footprint_boxes<T, D>(jb, r, f, i, i + 1, id, j);
+    const bool mul = merge && form_roulette(jb.form) == 0;
+    const double vol = double(r.vol[i]);
+    for (int k = 0; k < mb; ++k) {
+        const double m = r.marg[size_t(i) * mb + k];
+        f.marg[size_t(id) * mb + k] = mul ? 0.0 + vol * m : m;
     }
-    if (merge && form_roulette(jb.form) == 0) {
-        if (mb == 3)
-            merge_marginals<T, 3>(r, f, i, e, id);
-        else if (mb == 9)
-            merge_marginals<T, 9>(r, f, i, e, id);
-        else
-            merge_marginals<T, 27>(r, f, i, e, id);
-        f.scale[id] = 1.0;
-    } else {
-        for (int k = 0; k < mb; ++k) f.marg[size_t(id) * mb + k] = r.marg[size_t(i) * mb + k];
-        f.scale[id] = double(r.vol[i]);
+    f.scale[id] = mul ? 1.0 : vol;
+}
+
+/* 16 lanes per region that starts a footprint of merged regions (equal bin-dim codes):
+   lane k sums marginal entry k (and 16 + k with three bin dims), vol_r * marginal_r in
+   region order, FOOT_AHEAD regions' loads in flight.  A thread per footprint summing all
+   entries was one load latency per region: 215 us for 293 footprints of 10,000 regions,
+   here 52. */
+constexpr int FOOT_LANES = 16, FOOT_AHEAD = 8;
+template <typename T, int D>
+__global__ void __launch_bounds__(256) k_footprints(const Job<T>* __restrict__ jobs, RegionArrays<T> r, FootArrays<T> f,
+                                                    uint32_t n, int mb) {
+    const uint64_t gt = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const uint32_t i = uint32_t(gt / FOOT_LANES);
+    const int lane = int(threadIdx.x % FOOT_LANES), group = int(threadIdx.x % 64) / FOOT_LANES;
+    const bool starts = i < n && r.fpflag[i] != 0;
+    // the end of the run: the next region that starts a footprint (fpflag[n] is 0: n ends it)
+    uint32_t e = starts ? i + 1 : n;
+    bool open = starts && e < n;
+    while (__any(open)) {
+        const uint32_t p = e + uint32_t(lane);
+        const bool stop = open && (p >= n || r.fpflag[p] != 0);
+        const uint32_t m = uint32_t(__ballot(stop) >> (group * FOOT_LANES)) & ((1u << FOOT_LANES) - 1u);
+        if (open) {
+            e += m ? uint32_t(__ffs(int(m)) - 1) : uint32_t(FOOT_LANES);
+            open = m == 0;
+        }
     }
+    if (!starts) return;
+    const uint32_t id = r.fpid[i], j = r.job[i];
+    const Job<T>& jb = jobs[j];
+    if (lane == 0) footprint_boxes<T, D>(jb, r, f, i, e, id, j);
+    const bool mul = form_roulette(jb.form) == 0;
+    for (int k = lane; k < mb; k += FOOT_LANES) {
+        double acc = 0.0;
+        if (mul) {
+            for (uint32_t q0 = i; q0 < e; q0 += FOOT_AHEAD) {
+                double v[FOOT_AHEAD], m[FOOT_AHEAD];
+#pragma unroll
+                for (int u = 0; u < FOOT_AHEAD; ++u) {
+                    const uint32_t q = q0 + uint32_t(u) < e ? q0 + uint32_t(u) : i;
+                    v[u] = double(r.vol[q]);
+                    m[u] = r.marg[size_t(q) * mb + k];
+                }
+#pragma unroll
+                for (int u = 0; u < FOOT_AHEAD; ++u)
+                    if (q0 + uint32_t(u) < e) acc += v[u] * m[u];
+            }
+        } else {
+            acc = r.marg[size_t(i) * mb + k];
+        }
+        f.marg[size_t(id) * mb + k] = acc;
+    }
+    if (lane == 0) f.scale[id] = mul ? 1.0 : double(r.vol[i]);
 }
 
 /* *total += sum of x[0..n) in 64 bits.  The per-bin list offsets are 32-bit scans of
@@ -1698,39 +1733,83 @@ __device__ inline uint32_t div_fix(uint32_t c, uint32_t n, float inv) {
     return q;
 }
 
-/* Per-bin footprint lists by counting sort, one wave per footprint walking its pixel
-   box with the last bin dim fastest (consecutive lanes, consecutive bins).  Pair c of
-   footprint w is pair pofs[w] + c of the call.
+/* Per-bin footprint lists by counting sort, a lane per (bin, footprint) pair: pair c of
+   footprint w is pair pofs[w] + c of the call, its pixel box walked with the last bin dim
+   fastest (consecutive lanes, consecutive bins).
    PLACE = false: the pair's rank in its bin, rank = cnt[bin]++ (arrival order).
    PLACE = true (off = the counts' exclusive scan): each footprint id goes to
    off[bin] + rank, so every list is filled, in arrival order, with no atomics;
    k_sort_lists then puts each list in ascending footprint id (region order), which
-   fixes the per-bin summation order. */
+   fixes the per-bin summation order.
+   A wave takes BIN_PASS_RUN consecutive pairs.  Footprints run from one bin to the whole
+   image, and a wave per footprint left the largest one to a single wave: with 293
+   footprints of 1.07 M pairs the two passes took 605 + 577 us, here 11 + 14; with 262,144 of
+   16.9 M pairs 130 + 148, here 101 + 109. */
+constexpr uint32_t BIN_PASS_RUN = 256;
 template <typename T, bool PLACE>
-__global__ void k_bin_pass(const Job<T>* __restrict__ jobs, FootArrays<T> f, const uint32_t* __restrict__ nfp_ptr,
-                           uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off, uint32_t* __restrict__ lst,
-                           const uint32_t* __restrict__ pofs, uint32_t* __restrict__ rank) {
-    const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) / 64;
+__global__ void __launch_bounds__(256)
+    k_bin_pass(const Job<T>* __restrict__ jobs, FootArrays<T> f, const uint32_t* __restrict__ nfp_ptr,
+               uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off, uint32_t* __restrict__ lst,
+               const uint32_t* __restrict__ pofs, uint32_t* __restrict__ rank, uint32_t pairs) {
     const uint32_t lane = threadIdx.x % 64;
-    if (w >= *nfp_ptr) return;
-    const Job<T>& jb = jobs[f.job[w]];
-    const uint32_t* bx = f.box + size_t(w) * 6;
-    const uint32_t n0 = bx[1] - bx[0], n1 = bx[3] - bx[2], n2 = bx[5] - bx[4];
-    const uint32_t total = f.npairs[w];
-    const uint64_t r1 = jb.db > 1 ? jb.res[1] : 1, r2 = jb.db > 2 ? jb.res[2] : 1;
-    const float i2 = 1.0f / float(n2), i12 = 1.0f / float(n1);
-    uint32_t* const rk = rank + pofs[w];
-    for (uint32_t c = lane; c < total; c += 64) {
-        const uint32_t q2 = div_fix(c, n2, i2);  // c = (a0 * n1 + a1) * n2 + a2
+    const uint64_t first = (uint64_t(blockIdx.x) * (blockDim.x / 64) + threadIdx.x / 64) * BIN_PASS_RUN;
+    if (first >= pairs) return;
+    const uint32_t q_end = pairs - uint32_t(first) < BIN_PASS_RUN ? pairs : uint32_t(first) + BIN_PASS_RUN;
+    const uint32_t nfp = *nfp_ptr;
+    // the last footprint at or before the run's first pair, 64 probes at a time
+    uint32_t w = 0;
+    for (uint32_t n = nfp; n > 1;) {
+        const uint32_t step = (n + 63) / 64, i = lane * step;
+        const bool le = i < n && pofs[w + i] <= uint32_t(first);
+        const uint32_t c = uint32_t(__popcll(__ballot(le)));  // >= 1: pofs[w] is
+        w += (c - 1) * step;
+        n = n - (c - 1) * step < step ? n - (c - 1) * step : step;
+    }
+    for (uint32_t k = 0; k < q_end - uint32_t(first); k += 64) {
+        const uint32_t q0 = uint32_t(first) + k;
+        // every footprint has a pair, so 64 pairs from footprint w on lie in 64 footprints
+        const uint32_t start = w + lane < nfp ? pofs[w + lane] : 0xFFFFFFFFu;
+        const uint32_t q = q0 + lane;
+        uint32_t pos = 0;
+#pragma unroll
+        for (uint32_t b = 32; b > 0; b >>= 1) {
+            const uint32_t v = __shfl(start, int(pos + b), 64);
+            if (v <= q) pos += b;  // pos + b <= 63
+        }
+        const uint32_t c = q - __shfl(start, int(pos), 64), fi = w + pos;
+        // the footprint of the next 64's first pair
+        const uint32_t last = uint32_t(__builtin_amdgcn_readlane(int(pos), 63));
+        const uint32_t next = last < 63 ? uint32_t(__builtin_amdgcn_readlane(int(start), int(last) + 1))
+                                        : (w + 64 < nfp ? pofs[w + 64] : 0xFFFFFFFFu);
+        w += last + (next <= q0 + 64 ? 1u : 0u);
+        if (q >= q_end) break;
+        const uint2* bx = reinterpret_cast<const uint2*>(f.box + size_t(fi) * 6);
+        const uint2 b0 = bx[0], b1 = bx[1], b2 = bx[2];
+        const uint32_t n1 = b1.y - b1.x, n2 = b2.y - b2.x;
+        uint32_t jr1, jr2, jbase;
+        {
+            const uint32_t j = f.job[fi], j0 = __builtin_amdgcn_readfirstlane(j);
+            const Job<T>* jb = jobs + j0;  // one job's scalars for the whole wave, nearly always
+            jr1 = jb->db > 1 ? uint32_t(jb->res[1]) : 1u;
+            jr2 = jb->db > 2 ? uint32_t(jb->res[2]) : 1u;
+            jbase = uint32_t(jb->bin_base);
+            if (j != j0) {
+                jb = jobs + j;
+                jr1 = jb->db > 1 ? uint32_t(jb->res[1]) : 1u;
+                jr2 = jb->db > 2 ? uint32_t(jb->res[2]) : 1u;
+                jbase = uint32_t(jb->bin_base);
+            }
+        }
+        const uint32_t q2 = n2 == 1 ? c : div_fix(c, n2, 1.0f / float(n2));  // c = (a0 * n1 + a1) * n2 + a2
         const uint32_t a2 = c - q2 * n2;
-        const uint32_t a0 = div_fix(q2, n1, i12);
+        const uint32_t a0 = n1 == 1 ? q2 : div_fix(q2, n1, 1.0f / float(n1));
         const uint32_t a1 = q2 - a0 * n1;
-        const uint64_t local = (uint64_t(bx[0] + a0) * r1 + (bx[2] + a1)) * r2 + (bx[4] + a2);
-        const uint64_t bin = jb.bin_base + local;
+        // a batch's bins (and so their indexes) fit 32 bits
+        const uint32_t bin = jbase + ((b0.x + a0) * jr1 + (b1.x + a1)) * jr2 + (b2.x + a2);
         if constexpr (PLACE) {
-            lst[off[bin] + rk[c]] = w;
+            lst[off[bin] + rank[q]] = fi;
         } else {
-            rk[c] = atomicAdd(&cnt[bin], 1u);
+            rank[q] = atomicAdd(&cnt[bin], 1u);
         }
     }
 }

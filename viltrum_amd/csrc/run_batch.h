@@ -702,7 +702,12 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     size_t bytes = scan_reg_bytes;
     HIP_CHECK(hipError_t(rocprim::exclusive_scan(d_scan_tmp, bytes, ra.fpflag, ra.fpid, 0u, size_t(n_reg + 1),
                                                 rocprim::plus<uint32_t>(), st)));
-    vmx::k_footprints<T, D><<<reg_blocks, 256, 0, st>>>(d_jobs, ra, fa, uint32_t(n_reg), mb_max, merge);
+    // with bins along every dim no two regions share their bin-dim codes: nothing merges
+    if (merge && jobs[0].db < D)
+        vmx::k_footprints<T, D><<<unsigned((n_reg * vmx::FOOT_LANES + 255) / 256), 256, 0, st>>>(d_jobs, ra, fa,
+                                                                                            uint32_t(n_reg), mb_max);
+    else
+        vmx::k_footprints1<T, D><<<reg_blocks, 256, 0, st>>>(d_jobs, ra, fa, uint32_t(n_reg), mb_max, merge);
     HIP_CHECK(hipGetLastError());
     const uint32_t* d_nfp = ra.fpid + n_reg;
     // per-bin footprint lists: pairs emitted per footprint at scanned offsets, then a
@@ -782,17 +787,17 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     double* d_rrw = any_rr ? cp.take<double>(size_t(pairs) + 1) : nullptr;
     void* d_scan_bins_tmp = cp.take<char>(scan_bins_bytes + 256);
     HIP_CHECK(hipMemsetAsync(d_cnt, 0, sizeof(uint32_t) * (total_bins + 2), st));
-    const unsigned fp_blocks = unsigned((uint64_t(nfp) * 64 + 255) / 256);
+    const unsigned pass_blocks = unsigned((uint64_t(pairs) + 4 * vmx::BIN_PASS_RUN - 1) / (4 * vmx::BIN_PASS_RUN));
     if (pairs > 0)
-        vmx::k_bin_pass<T, false><<<fp_blocks, 256, 0, st>>>(d_jobs, fa, d_nfp, d_cnt, nullptr, nullptr, d_pofs,
-                                                             d_lst_tmp);
+        vmx::k_bin_pass<T, false><<<pass_blocks, 256, 0, st>>>(d_jobs, fa, d_nfp, d_cnt, nullptr, nullptr, d_pofs,
+                                                               d_lst_tmp, pairs);
     bytes = scan_bins_bytes;
     HIP_CHECK(hipError_t(rocprim::exclusive_scan(d_scan_bins_tmp, bytes, d_cnt, d_off, 0u, size_t(total_bins + 1),
                                                 rocprim::plus<uint32_t>(), st)));
     if (pairs > 0) {
         // the pairs' ranks live in d_lst_tmp until k_sort_long reuses it
-        vmx::k_bin_pass<T, true><<<fp_blocks, 256, 0, st>>>(d_jobs, fa, d_nfp, d_cnt, d_off, d_lst, d_pofs,
-                                                            d_lst_tmp);
+        vmx::k_bin_pass<T, true><<<pass_blocks, 256, 0, st>>>(d_jobs, fa, d_nfp, d_cnt, d_off, d_lst, d_pofs,
+                                                              d_lst_tmp, pairs);
         vmx::k_sort_lists<T><<<unsigned((total_bins + 255) / 256), 256, 0, st>>>(d_off, total_bins, d_lst, d_qlong,
                                                                                  fa, lp);
         vmx::k_sort_long<<<1024, 256, 0, st>>>(d_off, d_qlong, d_lst, d_lst_tmp);
