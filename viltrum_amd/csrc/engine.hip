@@ -342,12 +342,25 @@ void nn_forward(int kp, const float* params, const uint16_t* X, uint64_t n, floa
     HIP_CHECK(hipGetLastError());
 }
 
-void nn_grad(int kp, const float* params, const uint16_t* X, const float* tg, const uint32_t* idx, uint32_t count,
+/* The images a training step reads (nn::TrainNet), built from FP32 parameters. */
+void* pack_train(vmx_ctx* ctx, int kp, const float* params, hipStream_t st) {
+    void* out = nullptr;
+    with_kp(kp, [&](auto K) {
+        constexpr int KP = decltype(K)::value;
+        out = ensure(ctx->tr_net, sizeof(vmx::nn::TrainNet<KP>));
+        vmx::nn::k_pack_train<KP><<<1, 256, 0, st>>>(params, static_cast<vmx::nn::TrainNet<KP>*>(out));
+    });
+    HIP_CHECK(hipGetLastError());
+    return out;
+}
+
+void nn_grad(int kp, const void* images, const uint16_t* X, const float* tg, const uint32_t* idx, uint32_t count,
              float inv_batch, float* part, float* loss, int want_grad, hipStream_t st) {
     with_kp(kp, [&](auto K) {
         constexpr int KP = decltype(K)::value;
         const unsigned blocks = (count + 63) / 64;
-        vmx::nn::k_mlp_grad<KP><<<blocks, 256, 0, st>>>(params, X, tg, idx, count, inv_batch, part, loss, want_grad);
+        vmx::nn::k_mlp_grad<KP><<<blocks, vmx::nn::TRAIN_THREADS, 0, st>>>(
+            static_cast<const vmx::nn::TrainNet<KP>*>(images), X, tg, idx, count, inv_batch, part, loss, want_grad);
     });
     HIP_CHECK(hipGetLastError());
 }
@@ -493,6 +506,7 @@ void train_net(vmx_ctx* ctx, int dim, uint64_t count, const vmx_train_opts& o, v
     std::vector<float> lh(steps * nblk);
     double first = 0, last = 0;
     std::vector<uint32_t> tr(perm.begin(), perm.begin() + n_train);
+    void* images = pack_train(ctx, kp, d_p, st);
     for (uint32_t e = 0; e < epochs; ++e) {
         std::shuffle(tr.begin(), tr.end(), rng);
         HIP_CHECK(hipMemcpyAsync(d_idx, tr.data(), sizeof(uint32_t) * n_train, hipMemcpyHostToDevice, st));
@@ -500,13 +514,17 @@ void train_net(vmx_ctx* ctx, int dim, uint64_t count, const vmx_train_opts& o, v
         for (uint64_t s = 0; s < steps; ++s, ++t) {
             const uint64_t off = s * batch;
             const uint32_t cnt = uint32_t(std::min<uint64_t>(batch, n_train - off));
-            nn_grad(kp, d_p, X, tg, d_idx + off, cnt, 1.f / float(cnt), d_part, d_loss + s * nblk, 1, st);
+            nn_grad(kp, images, X, tg, d_idx + off, cnt, 1.f / float(cnt), d_part, d_loss + s * nblk, 1, st);
             const double frac = double(t) / total_steps;
             const float lr = float(lr0 * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(3.141592653589793 * frac))));
             const float c1 = float(1.0 / (1.0 - std::pow(double(b1), double(t + 1))));
             const float c2 = float(1.0 / (1.0 - std::pow(double(b2), double(t + 1))));
-            k_adam<<<unsigned((P + 255) / 256), 256, 0, st>>>(d_p, d_m, d_v, d_part, (cnt + 63) / 64, uint32_t(P), lr,
-                                                              b1, b2, 1e-8f, c1, c2);
+            with_kp(kp, [&](auto K) {
+                constexpr int KP = decltype(K)::value;
+                k_adam<KP><<<unsigned((P + 63) / 64), 64, 0, st>>>(d_p, d_m, d_v, d_part,
+                                                                   static_cast<TrainNet<KP>*>(images), (cnt + 63) / 64,
+                                                                   uint32_t(P), lr, b1, b2, 1e-8f, c1, c2);
+            });
             HIP_CHECK(hipGetLastError());
         }
         HIP_CHECK(hipMemcpyAsync(lh.data(), d_loss, sizeof(float) * steps * nblk, hipMemcpyDeviceToHost, st));
@@ -519,7 +537,7 @@ void train_net(vmx_ctx* ctx, int dim, uint64_t count, const vmx_train_opts& o, v
     }
     const double ms_train = ms_since(t0);
     // held-out loss
-    nn_grad(kp, d_p, X, tg, d_idx + n_train, uint32_t(n_valid), 1.f / float(n_valid), d_part, d_loss, 0, st);
+    nn_grad(kp, images, X, tg, d_idx + n_train, uint32_t(n_valid), 1.f / float(n_valid), d_part, d_loss, 0, st);
     std::vector<float> vl(vblk);
     HIP_CHECK(hipMemcpyAsync(vl.data(), d_loss, sizeof(float) * vblk, hipMemcpyDeviceToHost, st));
     HIP_CHECK(hipStreamSynchronize(st));
@@ -780,7 +798,8 @@ void vmx_ctx_destroy(vmx_ctx* ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     for (vmx_ctx::Buf* b : {&ctx->tree, &ctx->regs, &ctx->lists, &ctx->misc, &ctx->params, &ctx->bins, &ctx->bins2,
-                            &ctx->tr_x, &ctx->tr_t, &ctx->tr_idx, &ctx->tr_part, &ctx->tr_loss, &ctx->tr_state})
+                            &ctx->tr_x, &ctx->tr_t, &ctx->tr_idx, &ctx->tr_part, &ctx->tr_loss, &ctx->tr_state,
+                            &ctx->tr_net})
         if (b->p) (void)hipFree(b->p);
     for (vmx_ctx::Buf& b : ctx->nn)
         if (b.p) (void)hipFree(b.p);
@@ -1080,7 +1099,7 @@ int vmx_refiner_grad(vmx_ctx* ctx, int32_t dim, const float* params, uint64_t n,
         float* d_part = static_cast<float*>(ensure(ctx->tr_part, sizeof(float) * nblk * P));
         float* d_loss = static_cast<float*>(ensure(ctx->tr_loss, sizeof(float) * nblk));
         float* d_grad = static_cast<float*>(ensure(ctx->params, sizeof(float) * P));
-        nn_grad(kp, in.p, in.X, in.t, in.idx, uint32_t(n), 1.f / float(n), d_part, d_loss, 1, ctx->stream);
+        nn_grad(kp, pack_train(ctx, kp, in.p, ctx->stream), in.X, in.t, in.idx, uint32_t(n), 1.f / float(n), d_part, d_loss, 1, ctx->stream);
         vmx::nn::k_sum_parts<<<unsigned((P + 255) / 256), 256, 0, ctx->stream>>>(d_part, nblk, uint32_t(P), d_grad);
         HIP_CHECK(hipGetLastError());
         std::vector<float> lh(nblk);

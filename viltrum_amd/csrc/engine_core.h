@@ -54,7 +54,7 @@ struct vmx_ctx {
     Buf nn[VMX_MAX_DIM + 1];                       // FP32 priority-network parameters per dim
     Buf nn_lds[VMX_MAX_DIM + 1];                   // ... and their LDS image (nn::NetW<KP>)
     bool nn_ok[VMX_MAX_DIM + 1] = {};
-    Buf tr_x, tr_t, tr_idx, tr_part, tr_loss, tr_state;  // training work space
+    Buf tr_x, tr_t, tr_idx, tr_part, tr_loss, tr_state, tr_net;  // training work space
     hipEvent_t ev[8] = {};
     void* pinned = nullptr;  // host staging for small device-to-host readbacks
     size_t pinned_bytes = 0;

@@ -103,7 +103,7 @@ struct GrowLds {
         uint32_t hist[GROW_BUCKETS];  // low half: known nodes, high half: the pool
         T pool_b[S::POOL];
         uint32_t pool_s[S::POOL];  // node | split dim << 16
-        uint32_t list[S::SPLITS];
+        uint32_t list[2 * S::SPLITS];
         T box[S::SPLITS][2 * D];   // of the nodes split in a step: lo, hi
         // the node values of a step's children, as they go to memory; with the learned
         // priority a wave's 64 children use its part of net.act
@@ -138,8 +138,6 @@ struct GrowLds {
     int32_t last;
 };
 
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-
 /* A wave's 64 rows of features (`act`, rows of nn::WS) through the network; lane l gets
    row l's raw output.  tiles: 16-row tiles that hold rows in use (uniform).  The operands
    and their order are those of nn::forward_rows; the weights are the first operand, so a
@@ -171,13 +169,13 @@ __device__ inline float forward_wave(const nn::NetW<KP>& n, uint16_t* act, int t
 #pragma unroll
                 for (int k = 0; k < K / 32; ++k)
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k], x[q][k], acc, 0, 0, 0);
-                bf16x4_t h;
+                nn::bf16x4_t h;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float z = acc[i] + bv[i];
                     h[i] = __bf16(z > 0.f ? z : 0.f);  // round to nearest even, as nn::f2bf
                 }
-                *reinterpret_cast<bf16x4_t*>(act + (q * 16 + r) * nn::WS + f0) = h;
+                *reinterpret_cast<nn::bf16x4_t*>(act + (q * 16 + r) * nn::WS + f0) = h;
             }
         }
         team_sync<64>();
@@ -797,9 +795,11 @@ __global__ void __launch_bounds__(GROW_THREADS)
             pb[i] = q < np ? L.g.pool_b[q] : T(0);
             ps[i] = q < np ? L.g.pool_s[q] : NONE;
         }
-        // every wave busy until the end is near, then half: fewer splits too many
-        const bool all = g.deepen || need > (count - 1) / 2 + 2 * uint32_t(S::SPLITS);
-        grow_thresholds<T, D, LEARN>(L, need, uint32_t(S::SPLITS) / (all ? 1u : 2u));
+        // every wave busy until the end is near, then half: fewer splits too many; deepened
+        // steps take two passes of splits, whose children wait for the next step
+        const bool all = need > (count - 1) / 2 + 2 * uint32_t(S::SPLITS);
+        const uint32_t most = uint32_t(S::SPLITS) * (g.deepen ? 2u : 1u);
+        grow_thresholds<T, D, LEARN>(L, need, all ? most : most / 2);
         done = np == 0;
         if (done || np >= stop) break;  // uniform
         const T th = L.kb != NONE ? keys.lower(L.kb) : T(-INFINITY), tau = keys.lower(L.kt);
@@ -810,7 +810,7 @@ __global__ void __launch_bounds__(GROW_THREADS)
             const bool have = ps[i] != NONE;
             bool split = have && pb[i] >= eff;
             const uint32_t at = wave_append(split, &L.nlist[par]);
-            if (split && at >= uint32_t(S::SPLITS)) split = false;  // the rest of tau's bucket waits
+            if (split && at >= most) split = false;  // the rest of tau's bucket waits
             if (split) L.g.list[at] = ps[i];
             const bool keep = have && !split && pb[i] >= th;
             const uint32_t k = wave_append(keep, &L.npool[par ^ 1]);
@@ -822,7 +822,7 @@ __global__ void __launch_bounds__(GROW_THREADS)
             }
         }
         __syncthreads();
-        const uint32_t nl = L.nlist[par] < uint32_t(S::SPLITS) ? L.nlist[par] : uint32_t(S::SPLITS);
+        const uint32_t listed = L.nlist[par] < most ? L.nlist[par] : most;
         const uint32_t kept = L.npool[par ^ 1];
         par ^= 1;
         if (tid == 0) {  // the counters the next step fills
@@ -830,143 +830,147 @@ __global__ void __launch_bounds__(GROW_THREADS)
             L.npool[par ^ 1] = L.nnew[par ^ 1] = 0;
         }
         // room for the children, in the tree and in the pool (uniform)
-        if (count + 2 * nl > cap) {
-            if (tid == 0) L.flags |= count + 2 * nl > jb.node_cap ? JF_CAPACITY : 0u;
+        if (count + 2 * listed > cap) {
+            if (tid == 0) L.flags |= count + 2 * listed > jb.node_cap ? JF_CAPACITY : 0u;
             break;
         }
-        if (kept + 2 * nl > uint32_t(S::POOL)) break;
+        if (kept + 2 * listed > uint32_t(S::POOL)) break;
         ++steps;
-        // the children's node values gather in LDS as they go to memory, every lane at work
-        // whichever child a node is of: the planes they inherit (consecutive lanes,
-        // consecutive nodes), then the new ones (a handful of splits would else evaluate
-        // 3^(D-1) nodes one after the other).  A lane per child loads the rest meanwhile.
-        constexpr uint32_t KM = uint32_t(pow3(D - 1));
-        const uint32_t it = uint32_t(tid) / 2u;
-        const int c = tid & 1;
-        const bool go = it < nl;
-        const uint32_t entry = go ? L.g.list[it] : 0u;
-        const uint32_t node = base + (entry & 0xFFFFu);
-        T plo[D], phi[D], bp = T(0), b1p = T(0), errp = T(0);
-        uint32_t pcode[D];
-        if (go) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                plo[d] = t.lo[size_t(node) * D + d];
-                phi[d] = t.hi[size_t(node) * D + d];
-                pcode[d] = t.code[size_t(node) * D + d];
-            }
-            bp = t.b[node];
-            b1p = t.b1[node];
-            if constexpr (LEARN) errp = t.err[node];
-        }
-        for (uint32_t q0 = uint32_t(tid); q0 < nl * 4u * KM; q0 += 4u * uint32_t(NT)) {
-            T val[4];
-            T* at[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {  // four loads in flight
-                const uint32_t q = q0 + uint32_t(u * NT);
-                at[u] = nullptr;
-                if (q >= nl * 4u * KM) continue;
-                const uint32_t ci = q / (2u * KM), en = L.g.list[ci / 2u];
-                const int j0 = int(q % KM), far = int(q / KM) & 1, dim = int(en >> 16);  // plane 0 or 2 of the child
-                at[u] = L.child_values(ci) + Child<T, D>::at(2 * far, j0, dim);
-                val[u] = t.v[(size_t(base) + (en & 0xFFFFu)) * K + Child<T, D>::at(int(ci & 1u) + far, j0, dim)];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (at[u]) *at[u] = val[u];
-        }
-        if (go && c == 0) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                L.g.box[it][d] = plo[d];
-                L.g.box[it][D + d] = phi[d];
-            }
-        }
-        lds_barrier();
-        for (uint32_t q = uint32_t(tid); q < nl * 2u * KM; q += uint32_t(NT)) {
-            const uint32_t ci = q / KM;
-            const int dim = int(L.g.list[ci / 2u] >> 16);
-            T lo[D], hi[D], x[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                lo[d] = L.g.box[ci / 2u][d];
-                hi[d] = L.g.box[ci / 2u][D + d];
-            }
-            split_new_node<T, D>(lo, hi, dim, int(ci & 1u), int(q % KM), x);
-            L.child_values(ci)[Child<T, D>::at(1, int(q % KM), dim)] = f.template eval<Ahead<M>, D>(x);
-        }
-        lds_barrier();
-        if (uint32_t(wave) * 32u < nl) {
-            const size_t s = size_t(base) + count + 2 * it + c;
-            Child<T, D> ch;
-            T e = T(0), nb = T(0), nb1 = T(0);
-            int dm = 0, fd = 0;
-            float sc = 0.f;
-            bool pool = false;
-            uint16_t* row = nullptr;
-            if constexpr (LEARN) row = &L.g.net.act[wave][lane * nn::WS];
-            {
-                const uint32_t c0 = uint32_t(wave) * 64u, nc = 2u * nl - c0 < 64u ? 2u * nl - c0 : 64u;
-                const T* from = L.child_values(c0);
-                T* to = t.v + (size_t(base) + count + c0) * K;
-                for (uint32_t q = uint32_t(lane); q < nc * uint32_t(K); q += 64u) to[q] = from[q];
-            }
+        for (uint32_t l0 = 0; l0 < listed; l0 += uint32_t(S::SPLITS)) {
+            const uint32_t nl = listed - l0 < uint32_t(S::SPLITS) ? listed - l0 : uint32_t(S::SPLITS);
+            const uint32_t* list = L.g.list + l0;
+            // the children's node values gather in LDS as they go to memory, every lane at work
+            // whichever child a node is of: the planes they inherit (consecutive lanes,
+            // consecutive nodes), then the new ones (a handful of splits would else evaluate
+            // 3^(D-1) nodes one after the other).  A lane per child loads the rest meanwhile.
+            constexpr uint32_t KM = uint32_t(pow3(D - 1));
+            const uint32_t it = uint32_t(tid) / 2u;
+            const int c = tid & 1;
+            const bool go = it < nl;
+            const uint32_t entry = go ? list[it] : 0u;
+            const uint32_t node = base + (entry & 0xFFFFu);
+            T plo[D], phi[D], bp = T(0), b1p = T(0), errp = T(0);
+            uint32_t pcode[D];
             if (go) {
-                ch.box(plo, phi, int(entry >> 16), c);
-                ch.read(L.child_values(uint32_t(tid)));
-            }
-            team_sync<64>();  // learned: the features take the values' place
-            if (go) {
-                ch.score(jb.heur, e, dm);
-                if constexpr (LEARN) {
-                    if (jb.learn) ch.features(jb, pcode, row, sc, fd);
-                }
-            }
-            if constexpr (LEARN) {
-                if (jb.learn) {  // uniform; rows of lanes without a child hold what they held
-                    team_sync<64>();
-                    const uint32_t left = nl - uint32_t(wave) * 32u;
-                    const int tiles = __builtin_amdgcn_readfirstlane(left < 32u ? int(left + 7u) / 8 : 4);
-                    const float y = forward_wave<nn::Dims<D>::KP>(L.g.net.net, &L.g.net.act[wave][0], tiles, lane);
-                    if (go)
-                        learned_score<T, D>(y, L.g.net.net.mu, L.g.net.net.sigma, sc, fd, errp, jb.lfloor, pcode, ch.dim, c,
-                                            e, dm);
-                }
-            }
-            if (go) {
-                child_stack(e, bp, b1p, nb, nb1);
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
-                    const bool cut = d == ch.dim;
-                    if (cut && pcode[d] >= 0x80000000u) atomicOr(&L.flags, JF_DEPTH);
-                    const uint32_t code = cut ? pcode[d] * 2u + uint32_t(c) : pcode[d];
-                    deepest[d] = vmax(deepest[d], 31u - uint32_t(__clz(code)));
-                    t.lo[s * D + d] = ch.lo[d];
-                    t.hi[s * D + d] = ch.hi[d];
-                    t.code[s * D + d] = code;
+                    plo[d] = t.lo[size_t(node) * D + d];
+                    phi[d] = t.hi[size_t(node) * D + d];
+                    pcode[d] = t.code[size_t(node) * D + d];
                 }
-                t.err[s] = e;
-                t.dim[s] = dm;
-                t.b[s] = nb;
-                t.b1[s] = nb1;
-                t.parent[s] = int32_t(node);
-                t.child[s] = -1;
-                t.job[s] = j;
-                if (c == 0) t.child[node] = int32_t(s);
-                pool = nb >= th;
-                atomicAdd(&L.g.hist[grow_place(keys.bucket(nb))], pool ? 0x10001u : 1u);
+                bp = t.b[node];
+                b1p = t.b1[node];
+                if constexpr (LEARN) errp = t.err[node];
             }
-            const uint32_t k = kept + wave_append(pool, &L.nnew[par]);
-            if (pool) {
-                L.g.pool_b[k] = nb;
-                L.g.pool_s[k] = uint32_t(s - base) | uint32_t(dm) << 16;
+            for (uint32_t q0 = uint32_t(tid); q0 < nl * 4u * KM; q0 += 4u * uint32_t(NT)) {
+                T val[4];
+                T* at[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {  // four loads in flight
+                    const uint32_t q = q0 + uint32_t(u * NT);
+                    at[u] = nullptr;
+                    if (q >= nl * 4u * KM) continue;
+                    const uint32_t ci = q / (2u * KM), en = list[ci / 2u];
+                    const int j0 = int(q % KM), far = int(q / KM) & 1, dim = int(en >> 16);  // plane 0 or 2 of the child
+                    at[u] = L.child_values(ci) + Child<T, D>::at(2 * far, j0, dim);
+                    val[u] = t.v[(size_t(base) + (en & 0xFFFFu)) * K + Child<T, D>::at(int(ci & 1u) + far, j0, dim)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (at[u]) *at[u] = val[u];
             }
+            if (go && c == 0) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    L.g.box[it][d] = plo[d];
+                    L.g.box[it][D + d] = phi[d];
+                }
+            }
+            lds_barrier();
+            for (uint32_t q = uint32_t(tid); q < nl * 2u * KM; q += uint32_t(NT)) {
+                const uint32_t ci = q / KM;
+                const int dim = int(list[ci / 2u] >> 16);
+                T lo[D], hi[D], x[D];
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    lo[d] = L.g.box[ci / 2u][d];
+                    hi[d] = L.g.box[ci / 2u][D + d];
+                }
+                split_new_node<T, D>(lo, hi, dim, int(ci & 1u), int(q % KM), x);
+                L.child_values(ci)[Child<T, D>::at(1, int(q % KM), dim)] = f.template eval<Ahead<M>, D>(x);
+            }
+            lds_barrier();
+            if (uint32_t(wave) * 32u < nl) {
+                const size_t s = size_t(base) + count + 2 * it + c;
+                Child<T, D> ch;
+                T e = T(0), nb = T(0), nb1 = T(0);
+                int dm = 0, fd = 0;
+                float sc = 0.f;
+                bool pool = false;
+                uint16_t* row = nullptr;
+                if constexpr (LEARN) row = &L.g.net.act[wave][lane * nn::WS];
+                {
+                    const uint32_t c0 = uint32_t(wave) * 64u, nc = 2u * nl - c0 < 64u ? 2u * nl - c0 : 64u;
+                    const T* from = L.child_values(c0);
+                    T* to = t.v + (size_t(base) + count + c0) * K;
+                    for (uint32_t q = uint32_t(lane); q < nc * uint32_t(K); q += 64u) to[q] = from[q];
+                }
+                if (go) {
+                    ch.box(plo, phi, int(entry >> 16), c);
+                    ch.read(L.child_values(uint32_t(tid)));
+                }
+                team_sync<64>();  // learned: the features take the values' place
+                if (go) {
+                    ch.score(jb.heur, e, dm);
+                    if constexpr (LEARN) {
+                        if (jb.learn) ch.features(jb, pcode, row, sc, fd);
+                    }
+                }
+                if constexpr (LEARN) {
+                    if (jb.learn) {  // uniform; rows of lanes without a child hold what they held
+                        team_sync<64>();
+                        const uint32_t left = nl - uint32_t(wave) * 32u;
+                        const int tiles = __builtin_amdgcn_readfirstlane(left < 32u ? int(left + 7u) / 8 : 4);
+                        const float y = forward_wave<nn::Dims<D>::KP>(L.g.net.net, &L.g.net.act[wave][0], tiles, lane);
+                        if (go)
+                            learned_score<T, D>(y, L.g.net.net.mu, L.g.net.net.sigma, sc, fd, errp, jb.lfloor, pcode, ch.dim, c,
+                                                e, dm);
+                    }
+                }
+                if (go) {
+                    child_stack(e, bp, b1p, nb, nb1);
+#pragma unroll
+                    for (int d = 0; d < D; ++d) {
+                        const bool cut = d == ch.dim;
+                        if (cut && pcode[d] >= 0x80000000u) atomicOr(&L.flags, JF_DEPTH);
+                        const uint32_t code = cut ? pcode[d] * 2u + uint32_t(c) : pcode[d];
+                        deepest[d] = vmax(deepest[d], 31u - uint32_t(__clz(code)));
+                        t.lo[s * D + d] = ch.lo[d];
+                        t.hi[s * D + d] = ch.hi[d];
+                        t.code[s * D + d] = code;
+                    }
+                    t.err[s] = e;
+                    t.dim[s] = dm;
+                    t.b[s] = nb;
+                    t.b1[s] = nb1;
+                    t.parent[s] = int32_t(node);
+                    t.child[s] = -1;
+                    t.job[s] = j;
+                    if (c == 0) t.child[node] = int32_t(s);
+                    pool = nb >= th;
+                    atomicAdd(&L.g.hist[grow_place(keys.bucket(nb))], pool ? 0x10001u : 1u);
+                }
+                const uint32_t k = kept + wave_append(pool, &L.nnew[par]);
+                if (pool) {
+                    L.g.pool_b[k] = nb;
+                    L.g.pool_s[k] = uint32_t(s - base) | uint32_t(dm) << 16;
+                }
+            }
+            count += 2 * nl;
+            // the children's stores need not have landed yet: the barrier after the next
+            // step's filter orders them before any node of theirs is read
+            lds_barrier();
         }
-        count += 2 * nl;
-        // the children's stores need not have landed yet: the barrier after the next
-        // step's filter orders them before any node of theirs is read
-        lds_barrier();
     }
 #pragma unroll
     for (int d = 0; d < D; ++d)

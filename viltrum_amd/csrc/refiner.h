@@ -56,16 +56,6 @@ __device__ inline f32x4_t mm_tile(const uint16_t* a, int lda, const uint16_t* bt
     return acc;
 }
 
-/* Tile of A^T B over the sample dim: A[S][m] and B[S][n] both sample-major. */
-__device__ inline f32x4_t mm_tile_tn(const uint16_t* a, int lda, const uint16_t* b, int ldb, int S, int lane) {
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const int r = lane & 15, kq = (lane >> 4) * 8;
-    for (int s0 = 0; s0 < S; s0 += 32)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gather8(a + (s0 + kq) * lda + r, lda),
-                                                      gather8(b + (s0 + kq) * ldb + r, ldb), acc, 0, 0, 0);
-    return acc;
-}
-
 /* Forward weights in LDS. */
 template <int KP>
 struct alignas(16) NetW {  // size a multiple of 16 bytes (copied as 16-byte words)
@@ -125,12 +115,52 @@ __global__ void k_pack_net(const float* __restrict__ p, NetW<KP>* out) {
     load_net<KP>(*out, p);
 }
 
+/* What a training step reads: the forward image and the input-major copies, kept in device
+   memory beside the FP32 parameters and renewed by the optimizer (building them from the
+   parameters in every block was most of a step). */
+template <int KP>
+struct TrainNet {
+    NetW<KP> net;
+    NetWN n;
+};
+
 template <int KP>
 __device__ inline void load_net_n(NetWN& n, const float* __restrict__ p) {
     using L = Layout<KP>;
     for (int i = threadIdx.x; i < W * W; i += blockDim.x) {
         n.w1n[i / W][i % W] = f2bf(p[L::w1 + i]);
         n.w2n[i / W][i % W] = f2bf(p[L::w2 + i]);
+    }
+}
+
+template <int KP>
+__global__ void k_pack_train(const float* __restrict__ p, TrainNet<KP>* out) {
+    load_net<KP>(out->net, p);
+    load_net_n<KP>(out->n, p);
+}
+
+/* Parameter i of the flat array into the images. */
+template <int KP>
+__device__ inline void store_param(TrainNet<KP>& t, uint32_t i, float x) {
+    using L = Layout<KP>;
+    if (i < uint32_t(L::b0)) {
+        t.net.w0t[i % W][i / W] = f2bf(x);
+    } else if (i < uint32_t(L::w1)) {
+        t.net.b0[i - L::b0] = x;
+    } else if (i < uint32_t(L::b1)) {
+        const uint32_t q = i - L::w1;
+        t.net.w1t[q % W][q / W] = t.n.w1n[q / W][q % W] = f2bf(x);
+    } else if (i < uint32_t(L::w2)) {
+        t.net.b1[i - L::b1] = x;
+    } else if (i < uint32_t(L::b2)) {
+        const uint32_t q = i - L::w2;
+        t.net.w2t[q % W][q / W] = t.n.w2n[q / W][q % W] = f2bf(x);
+    } else if (i < uint32_t(L::w3)) {
+        t.net.b2[i - L::b2] = x;
+    } else if (i < uint32_t(L::b3)) {
+        t.net.w3[i - L::w3] = bf2f(f2bf(x));
+    } else {
+        t.net.b3 = x;
     }
 }
 
@@ -217,112 +247,196 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const float* __restrict__ p
 /* ---------------------------------------------------------------- training
    Gradient of 0.5 * sum_r c (y_r - (t_r - mu) / sigma)^2 over one 64-row tile per block
    (rows idx[blk*64 ..], c = inv_batch), written to part[blk][trained]; the block's loss
-   sum goes to loss[blk] (want_grad = 0: the loss only).  Deterministic: no atomics. */
+   sum goes to loss[blk] (want_grad = 0: the loss only).  Deterministic: no atomics.
+   A minibatch of 1024 rows is 16 blocks, one per CU and most of the chip idle, so a step is
+   its chain of layers: 16 waves take a 16x16 tile each (4 waves took four in turn), weights
+   come as images, and activations and deltas are kept both row-major and transposed (each
+   tile by two MFMAs, one per operand order, whose results a lane stores as 8 bytes), so
+   that every operand of the next product is one 16-byte read.  KP = 32: 37 us a step, now
+   10.5; KP = 288: 104, now 15.9.  Sums over the rows run in row order. */
+constexpr int TRAIN_THREADS = 1024;
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
 template <int KP>
-__global__ void __launch_bounds__(256) k_mlp_grad(const float* __restrict__ params, const uint16_t* __restrict__ X,
-                                                  const float* __restrict__ tgt, const uint32_t* __restrict__ idx,
-                                                  uint32_t count, float inv_batch, float* __restrict__ part,
-                                                  float* __restrict__ loss, int want_grad) {
+struct TrainLds {
+    // wide first layers (37 KB at KP = 288) are read from device memory
+    static constexpr bool W0_DEV = KP >= 128;
+    typename std::conditional<W0_DEV, NetTail, NetW<KP>>::type net;
+    NetWN n;
+    alignas(16) uint16_t xs[64][KP + 8];
+    alignas(16) uint16_t h[3][64][WS];   // [row][feature]
+    alignas(16) uint16_t ht[2][W][WS];   // [feature][row], layers 0 and 1
+    alignas(16) uint16_t g[2][64][WS];
+    alignas(16) uint16_t gt[2][W][WS];
+    float y[64], dy[64];
+};
+
+template <int KP>
+__global__ void __launch_bounds__(TRAIN_THREADS)
+    k_mlp_grad(const TrainNet<KP>* __restrict__ tn, const uint16_t* __restrict__ X, const float* __restrict__ tgt,
+               const uint32_t* __restrict__ idx, uint32_t count, float inv_batch, float* __restrict__ part,
+               float* __restrict__ loss, int want_grad) {
     using L = Layout<KP>;
-    __shared__ NetW<KP> net;
-    __shared__ NetWN netn;
-    __shared__ __attribute__((aligned(16))) uint16_t xs[64][KP + 8];
-    __shared__ __attribute__((aligned(16))) uint16_t h[3][64][WS];
-    __shared__ __attribute__((aligned(16))) uint16_t g[2][64][WS];
-    __shared__ float yo[64], dy[64];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nw = blockDim.x >> 6;
+    using LD = TrainLds<KP>;
+    __shared__ LD S;
+    constexpr int NT = TRAIN_THREADS, NW = NT / 64;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int r16 = lane & 15, q4 = (lane >> 4) * 4;
     const uint32_t base = blockIdx.x * 64u;
     float* out = part + size_t(blockIdx.x) * L::trained;
-    load_net<KP>(net, params);
-    load_net_n<KP>(netn, params);
-    for (int i = tid; i < 64 * KP; i += blockDim.x) {
-        const int r = i / KP, k = i % KP;
-        xs[r][k] = base + r < count ? X[size_t(idx[base + r]) * KP + k] : uint16_t(0);
+    {
+        constexpr size_t skip = LD::W0_DEV ? net_tail_offset<KP>() : 0;
+        const uint4* a = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(&tn->net) + skip);
+        uint4* d = reinterpret_cast<uint4*>(&S.net);
+        for (int i = tid; i < int(sizeof(S.net) / 16); i += NT) d[i] = a[i];
+        const uint4* a2 = reinterpret_cast<const uint4*>(&tn->n);
+        uint4* d2 = reinterpret_cast<uint4*>(&S.n);
+        for (int i = tid; i < int(sizeof(S.n) / 16); i += NT) d2[i] = a2[i];
+        constexpr int V = KP / 8;  // 16-byte pieces of a row (KP is a multiple of 32)
+        for (int i = tid; i < 64 * V; i += NT) {
+            const int r = i / V, k = i % V;
+            const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+            *reinterpret_cast<uint4*>(&S.xs[r][8 * k]) =
+                base + r < count ? reinterpret_cast<const uint4*>(X + size_t(idx[base + r]) * KP)[k] : z;
+        }
     }
+    float tg = 0.f;
+    if (tid < 64 && base + tid < count) tg = tgt[idx[base + tid]];
     __syncthreads();
-    forward_block<KP>(net, &xs[0][0], 64, &h[0][0][0], &h[1][0][0], &h[2][0][0], yo);
+    const uint16_t* w0t;
+    if constexpr (LD::W0_DEV)
+        w0t = &tn->net.w0t[0][0];
+    else
+        w0t = &S.net.w0t[0][0];
+    // forward: tile (rt, ct) of each layer to wave 4 rt + ct
+    const int rt = wave >> 2, ct = wave & 3;
+    auto layer = [&](const uint16_t* wt, int ldw, const float* bias, const uint16_t* x, int ldx, int K, uint16_t* h,
+                     uint16_t* ht) {
+        const uint16_t *xr = x + rt * 16 * ldx, *wr = wt + ct * 16 * ldw;
+        {  // a lane's four results: features ct * 16 + q4 + i of row rt * 16 + r16
+            const f32x4_t acc = mm_tile(wr, ldw, xr, ldx, K, lane);
+            bf16x4_t v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float z = acc[i] + bias[ct * 16 + q4 + i];
+                v[i] = __bf16(z > 0.f ? z : 0.f);
+            }
+            *reinterpret_cast<bf16x4_t*>(h + (rt * 16 + r16) * WS + ct * 16 + q4) = v;
+        }
+        if (ht) {  // rows rt * 16 + q4 + i of feature ct * 16 + r16
+            const f32x4_t acc = mm_tile(xr, ldx, wr, ldw, K, lane);
+            const float bv = bias[ct * 16 + r16];
+            bf16x4_t v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float z = acc[i] + bv;
+                v[i] = __bf16(z > 0.f ? z : 0.f);
+            }
+            *reinterpret_cast<bf16x4_t*>(ht + (ct * 16 + r16) * WS + rt * 16 + q4) = v;
+        }
+        __syncthreads();
+    };
+    static_assert(NW == 16, "a wave per tile of a layer");
+    layer(w0t, KP + 8, S.net.b0, &S.xs[0][0], KP + 8, KP, &S.h[0][0][0], &S.ht[0][0][0]);
+    layer(&S.net.w1t[0][0], WS, S.net.b1, &S.h[0][0][0], WS, W, &S.h[1][0][0], &S.ht[1][0][0]);
+    layer(&S.net.w2t[0][0], WS, S.net.b2, &S.h[1][0][0], WS, W, &S.h[2][0][0], nullptr);
+    dense_out(S.net.w3, S.net.b3, &S.h[2][0][0], 64, S.y);
+    __syncthreads();
     if (tid < 64) {
         float d = 0.f;
         if (base + tid < count) {
-            const float tn = (tgt[idx[base + tid]] - net.mu) / net.sigma;
-            d = yo[tid] - tn;
+            const float t = (tg - S.net.mu) / S.net.sigma;
+            d = S.y[tid] - t;
         }
-        dy[tid] = d * inv_batch;
-        yo[tid] = 0.5f * d * d * inv_batch;
+        S.dy[tid] = d * inv_batch;
+        S.y[tid] = 0.5f * d * d * inv_batch;
     }
     __syncthreads();
-    if (!want_grad) {  // loss only (validation)
-        if (tid == 0) {
-            float ls = 0.f;
-            for (int r = 0; r < 64; ++r) ls += yo[r];
+    if (wave == NW - 1) {  // the loss, and with it the output bias's gradient
+        if (lane == 0) {
+            float s = 0.f, ls = 0.f;
+#pragma unroll 16
+            for (int r = 0; r < 64; ++r) {
+                s += S.dy[r];
+                ls += S.y[r];
+            }
+            if (want_grad) out[L::b3] = s;
             loss[blockIdx.x] = ls;
         }
-        return;
     }
-    // output layer
-    if (tid < W) {
+    if (!want_grad) return;  // validation
+    if (wave == NW - 2) {  // output layer
         float s = 0.f;
-        for (int r = 0; r < 64; ++r) s += bf2f(h[2][r][tid]) * dy[r];
-        out[L::w3 + tid] = s;
-    } else if (tid == W) {
-        float s = 0.f, ls = 0.f;
-        for (int r = 0; r < 64; ++r) {
-            s += dy[r];
-            ls += yo[r];
-        }
-        out[L::b3] = s;
-        loss[blockIdx.x] = ls;
+#pragma unroll 16
+        for (int r = 0; r < 64; ++r) s += bf2f(S.h[2][r][lane]) * S.dy[r];
+        out[L::w3 + lane] = s;
     }
-    for (int i = tid; i < 64 * W; i += blockDim.x) {
-        const int r = i / W, k = i % W;
-        g[0][r][k] = bf2f(h[2][r][k]) > 0.f ? f2bf(dy[r] * net.w3[k]) : uint16_t(0);
+    {
+        const int r = tid >> 4, k0 = (tid & 15) * 4;  // four features of a row
+        uint16_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = bf2f(S.h[2][r][k0 + i]) > 0.f ? f2bf(S.dy[r] * S.net.w3[k0 + i]) : uint16_t(0);
+            S.g[0][r][k0 + i] = v[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S.gt[0][k0 + i][r] = v[i];
     }
     __syncthreads();
+    // sum over the rows, in row order, of feature `lane` of a transposed delta
+    auto bias_grad = [&](const uint16_t* gt, float* o) {
+        float s = 0.f;
+#pragma unroll
+        for (int r = 0; r < 64; r += 8) {
+            const u16x8_t v = *reinterpret_cast<const u16x8_t*>(gt + lane * WS + r);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s += bf2f(v[i]);
+        }
+        o[lane] = s;
+    };
+    // tile (mt, nt) of A^T B over the rows, both transposed
+    auto weight_grad = [&](const uint16_t* at, const uint16_t* bt, int mt, int nt, float* o) {
+        const f32x4_t acc = mm_tile(at + mt * 16 * WS, WS, bt + nt * 16 * WS, WS, 64, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[(mt * 16 + q4 + i) * W + nt * 16 + r16] = acc[i];
+    };
     // hidden layers 2 and 1: dW = h_in^T g, db = sum g, g_in = (g W^T) masked
-    for (int layer = 2; layer >= 1; --layer) {
-        const uint16_t* hin = &h[layer - 1][0][0];
-        const uint16_t* gl = &g[layer == 2 ? 0 : 1][0][0];
-        uint16_t* gnext = &g[layer == 2 ? 1 : 0][0][0];
-        const uint16_t* wn = layer == 2 ? &netn.w2n[0][0] : &netn.w1n[0][0];
-        const int ow = layer == 2 ? L::w2 : L::w1, ob = layer == 2 ? L::b2 : L::b1;
-        for (int u = wave; u < 16 + 16; u += nw) {
-            if (u < 16) {
-                const int mt = u / 4, nt = u % 4;
-                const f32x4_t acc = mm_tile_tn(hin + mt * 16, WS, gl + nt * 16, WS, 64, lane);
-                const int o = nt * 16 + (lane & 15);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[ow + (mt * 16 + (lane >> 4) * 4 + i) * W + o] = acc[i];
-            } else {
-                const int rt = (u - 16) / 4, ct = (u - 16) % 4;
-                const f32x4_t acc = mm_tile(gl + rt * 16 * WS, WS, wn + ct * 16 * WS, WS, W, lane);
-                const int k = ct * 16 + (lane & 15);
+    for (int l = 2; l >= 1; --l) {
+        const int cur = l == 2 ? 0 : 1, nxt = cur ^ 1;
+        const uint16_t *hin = &S.h[l - 1][0][0], *hint = &S.ht[l - 1][0][0];
+        const uint16_t *gl = &S.g[cur][0][0], *glt = &S.gt[cur][0][0];
+        const uint16_t* wn = l == 2 ? &S.n.w2n[0][0] : &S.n.w1n[0][0];
+        {
+            const uint16_t *gr = gl + rt * 16 * WS, *wr = wn + ct * 16 * WS;
+            const f32x4_t a = mm_tile(wr, WS, gr, WS, W, lane);  // inputs ct * 16 + q4 + i of row rt * 16 + r16
+            const f32x4_t b = mm_tile(gr, WS, wr, WS, W, lane);  // rows rt * 16 + q4 + i of input ct * 16 + r16
+            uint16_t* ga = &S.g[nxt][rt * 16 + r16][ct * 16 + q4];
+            uint16_t* gb = &S.gt[nxt][ct * 16 + r16][rt * 16 + q4];
+            const uint16_t* ha = hin + (rt * 16 + r16) * WS + ct * 16 + q4;
+            const uint16_t* hb = hint + (ct * 16 + r16) * WS + rt * 16 + q4;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = rt * 16 + (lane >> 4) * 4 + i;
-                    gnext[r * WS + k] = bf2f(hin[r * WS + k]) > 0.f ? f2bf(acc[i]) : uint16_t(0);
-                }
+            for (int i = 0; i < 4; ++i) {
+                ga[i] = bf2f(ha[i]) > 0.f ? f2bf(a[i]) : uint16_t(0);
+                gb[i] = bf2f(hb[i]) > 0.f ? f2bf(b[i]) : uint16_t(0);
             }
         }
-        if (tid < W) {
-            float s = 0.f;
-            for (int r = 0; r < 64; ++r) s += bf2f(gl[r * WS + tid]);
-            out[ob + tid] = s;
-        }
+        weight_grad(hint, glt, rt, ct, out + (l == 2 ? L::w2 : L::w1));
+        if (wave == l) bias_grad(glt, out + (l == 2 ? L::b2 : L::b1));
         __syncthreads();
     }
-    // input layer: dW0 = x^T g0 (g0 is in g[0] after the loop)
-    for (int u = wave; u < (KP / 16) * 4; u += nw) {
-        const int mt = u / 4, nt = u % 4;
-        const f32x4_t acc = mm_tile_tn(&xs[0][0] + mt * 16, KP + 8, &g[0][0][0] + nt * 16, WS, 64, lane);
-        const int o = nt * 16 + (lane & 15);
+    // input layer: dW0 = x^T g0 (g0 is in g[0] and gt[0] after the loop)
+    for (int u = wave; u < (KP / 16) * 4; u += NW) {
+        const int mt = u / 4, nt = u % 4, kq = (lane >> 4) * 8;
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[L::w0 + (mt * 16 + (lane >> 4) * 4 + i) * W + o] = acc[i];
+        for (int s0 = 0; s0 < 64; s0 += 32)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gather8(&S.xs[s0 + kq][mt * 16 + r16], KP + 8),
+                                                          ld8(&S.gt[0][nt * 16 + r16][s0 + kq]), acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[L::w0 + (mt * 16 + q4 + i) * W + nt * 16 + r16] = acc[i];
     }
-    if (tid < W) {
-        float s = 0.f;
-        for (int r = 0; r < 64; ++r) s += bf2f(g[0][r][tid]);
-        out[L::b0 + tid] = s;
-    }
+    if (wave == NW - 1) bias_grad(&S.gt[0][0][0], out + L::b0);
 }
 
 /* 64-bit FNV-1a over the 32-bit words of row i (kp BF16 features, then the target's
@@ -354,19 +468,31 @@ static __global__ void k_sum_parts(const float* __restrict__ part, uint32_t nblk
 }
 
 /* Adam (Kingma & Ba 2015) on the trained parameters; the gradient is the block-ordered
-   sum of the partials.  c1, c2 are the bias corrections 1/(1-beta^t). */
-static __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ part, uint32_t nblk, uint32_t P, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
+   sum of the partials, whose loads are all in flight at once.  c1, c2 are the bias
+   corrections 1/(1-beta^t).  The new values go into the images too. */
+template <int KP>
+__global__ void __launch_bounds__(64) k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
+                                             const float* __restrict__ part, TrainNet<KP>* __restrict__ tn, uint32_t nblk,
+                                             uint32_t P, float lr, float b1, float b2, float eps, float c1, float c2) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= P) return;
+    const float pi = p[i], m0 = m[i], v0 = v[i];
     float gsum = 0.f;
-    for (uint32_t b = 0; b < nblk; ++b) gsum += part[size_t(b) * P + i];
-    const float mi = b1 * m[i] + (1.f - b1) * gsum;
-    const float vi = b2 * v[i] + (1.f - b2) * gsum * gsum;
+    for (uint32_t b0 = 0; b0 < nblk; b0 += 16) {
+        float g[16];
+#pragma unroll
+        for (uint32_t u = 0; u < 16; ++u) g[u] = part[size_t(b0 + u < nblk ? b0 + u : 0u) * P + i];
+#pragma unroll
+        for (uint32_t u = 0; u < 16; ++u)
+            if (b0 + u < nblk) gsum += g[u];
+    }
+    const float mi = b1 * m0 + (1.f - b1) * gsum;
+    const float vi = b2 * v0 + (1.f - b2) * gsum * gsum;
     m[i] = mi;
     v[i] = vi;
-    p[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    const float x = pi - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    p[i] = x;
+    store_param<KP>(*tn, i, x);
 }
 
 }  // namespace nn
