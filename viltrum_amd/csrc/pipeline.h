@@ -46,6 +46,7 @@ struct Job {
     uint32_t N, node_base, node_cap, reg_base;
     uint32_t tile_base;  // first tile (of 256 bins) of this job in the per-bin kernel's grid
     uint32_t tile_base2;  // first tile of this job in the region-major per-bin kernel's grid
+    int32_t tiled;        // the per-bin kernel's tiles are 16 x 16 bins, else runs of 256
     int32_t db, mb, form, heur;
     int32_t learn;   // refinement priority from the network (refiner.h)
     int32_t lfloor;  // with learn: every dim is first halved lfloor times, widest first
@@ -1988,8 +1989,8 @@ __device__ inline uint32_t xcd_tile(uint32_t w, uint32_t G) {
    the polynomial's value at the sample depends on it, while the control-variate
    integral keeps pos_in). */
 
-/* One lane per bin (all jobs of the batch), one block per tile of 256 consecutive bins
-   of one job.  The lane sums the control variate over the
+/* One lane per bin (all jobs of the batch), one block per tile of 256 bins of one job
+   (16 x 16, or consecutive ones: bins_tiled).  The lane sums the control variate over the
    bin's footprints in list order (FP64), then draws the spp residual samples -- a region
    uniform among the bin's regions (binary search over footprint counts cached in LDS),
    a point uniform in bin x region -- and forms the estimator of the job's form
@@ -2017,6 +2018,22 @@ VMX_HD inline bool rm_job(int form, uint32_t N) {
    of 256 bins. */
 inline uint32_t rm_tiles(int db, const uint64_t* res, uint64_t nbins) {
     if (db == 2) return uint32_t(((res[0] + 15) / 16) * ((res[1] + 15) / 16));
+    return uint32_t((nbins + 255) / 256);
+}
+
+/* Whether a job's tiles in k_bins1 are 16 x 16 bins, 8 x 8 per wave: neighbours in both
+   dims share regions, so far more waves hold bins of one region each than with runs of a
+   row (an edge of small regions crosses every row, but few squares).  Narrow grids keep
+   runs of 256 bins (a square would stick out), and so does FP64, which has no loop for
+   single regions (301 x 217 bins of 20000 regions, 64 spp: 190 us in runs, 215 us in squares).  FP32, 64 integrals of 512 x 512 bins and 4096 regions, 16 spp: the
+   single-region loop in runs 1418 us, in squares 1232 us. */
+template <typename T>
+inline bool bins_tiled(int db, const uint64_t* res) {
+    return sizeof(T) == 4 && db == 2 && res[0] >= 16 && res[1] >= 16;
+}
+template <typename T>
+inline uint32_t bins_tiles(int db, const uint64_t* res, uint64_t nbins) {
+    if (bins_tiled<T>(db, res)) return uint32_t(((res[0] + 15) / 16) * ((res[1] + 15) / 16));
     return uint32_t((nbins + 255) / 256);
 }
 
@@ -2069,12 +2086,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
     __syncthreads();
     const F& f_lds = *reinterpret_cast<const F*>(f_raw);
     {
-        const uint64_t b = uint64_t(tile - jb.tile_base) * blockDim.x + tid;  // bin within the job
+        uint64_t b = uint64_t(tile - jb.tile_base) * blockDim.x + tid;  // bin within the job
+        uint32_t p[3] = {0, 0, 0};
+        const bool tiled = DB == 2 && jb.tiled;
+        if (tiled) {
+            const uint32_t tt = tile - jb.tile_base, r1 = uint32_t(jb.res[1]), across = (r1 + 15) / 16;
+            const uint32_t wave = uint32_t(tid) >> 6, lane = uint32_t(tid) & 63;
+            p[0] = (tt / across) * 16 + (wave >> 1) * 8 + lane / 8;
+            p[1] = (tt % across) * 16 + (wave & 1) * 8 + lane % 8;
+            if (p[0] >= uint32_t(jb.res[0]) || p[1] >= r1) return;
+            b = uint64_t(p[0]) * r1 + p[1];
+        }
         if (b >= jb.nbins) return;
         const uint64_t gb = jb.bin_base + b;
         const uint32_t o = off[gb], nf = off[gb + 1] - o;
-        uint32_t p[3] = {0, 0, 0};
-        {
+        if (!tiled) {
             uint32_t rem = uint32_t(b);  // a job holds at most 2^31 bins
 #pragma unroll
             for (int i = DB - 1; i >= 0; --i) {
@@ -2214,9 +2240,81 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
         T k_f = 0, k_a = 0;
         const uint64_t ns_run = sampling ? spp : 0;
         constexpr int SR = samp_stride<D>();
+        // One region per bin for the whole wave (regions of a bin's size or more, all but the
+        // bins that small regions cross): its box, inverse extents and coefficients stay in
+        // registers and no region is drawn, so a sample is its coordinates' draws, f, P and
+        // the moments.  The words drawn, and the arithmetic on them, are the general loop's.
+        // Bound by VALU issue, 128 instructions a sample here (Philox 29 multiply-adds a
+        // group, 9-10 per Gaussian); 202 a sample over all waves before, 169 now: 64
+        // integrals of 512 x 512 bins and 4096 regions at 16 spp 1608 -> 1232 us with the
+        // tiles of 16 x 16 bins, one such integral 64 -> 52 us.
+        bool general = true;
+        if constexpr (FP32 && MODE == 0 && !STRAT && D <= 2) {
+            if (__all((n == 1 && nf == 1) || ns_run == 0)) {
+                general = false;
+                const T* rec = r.samp + size_t(ns_run > 0 ? first0 : 0u) * SR;
+                T ilo[D], ihi[D], ext[D], rl[D], inv[D], coef[K];
+                bool empty = false;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    rl[d] = rec[d];
+                    ilo[d] = __builtin_fmaxf(blo[d], rl[d]);
+                    ihi[d] = __builtin_fmaxf(ilo[d], __builtin_fminf(bhi[d], rec[D + d]));
+                    if (ilo[d] >= ihi[d]) empty = true;
+                    ext[d] = ihi[d] - ilo[d];
+                    inv[d] = rec[2 * D + d];
+                }
+#pragma unroll
+                for (int k = 0; k < K; ++k) coef[k] = rec[3 * D + k];
+                const T vol = box_volume<T, D>(ilo, ihi);
+                const T w = wn * vol;
+                const bool alpha1 = jb.form == VMX_FORM_CV_ALPHA1;
+                const double a1v = a1w * double(vol);
+                for (uint64_t s0 = 0; s0 < ns_run; s0 += 4) {
+                    GroupDraws<T, D> u(uint32_t(s0 >> 2), b, jb.stream, jb.seed_lo, jb.seed_hi);
+                    const uint64_t left = ns_run - s0;
+                    T gf = 0, ga = 0, gmf = 0, gma = 0, gmaa = 0, gmfa = 0;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (uint64_t(k) >= left) break;
+                        T x[D], t[D];
+#pragma unroll
+                        for (int d = 0; d < D; ++d) {
+                            x[d] = mul_add<true>(u.coord(k, d), ext[d], ilo[d]);
+                            t[d] = (x[d] - rl[d]) * inv[d];
+                        }
+                        const T fx = residual_eval<M, D>(f_lds, x);
+                        const T px = eval_monomials<T, D, true>(coef, t);
+                        if (alpha1) {
+                            if (!empty) acc1 += double(fx - px) * a1v;
+                            continue;
+                        }
+                        const T fsv = fx * w, asv = px * w;
+                        if (k == 0 && s0 == 0) {  // the bin's first sample shifts the moments
+                            k_f = vabs(fsv);
+                            k_a = vabs(asv);
+                        }
+                        gf += fsv;
+                        ga += asv;
+                        const T df = vabs(fsv) - k_f, da = vabs(asv) - k_a;
+                        gmf += df;
+                        gma += da;
+                        gmaa += da * da;
+                        gmfa += df * da;
+                    }
+                    if (alpha1) continue;
+                    sf.add(gf);
+                    sa.add(ga);
+                    mf.add(gmf);
+                    ma.add(gma);
+                    maa.add(gmaa);
+                    mfa.add(gmfa);
+                }
+            }
+        }
         // samples in groups of 4: one draw per word type serves the group, and the
         // group's partial sums are compensated once
-        for (uint64_t s0 = 0; s0 < ns_run; s0 += 4) {
+        for (uint64_t s0 = 0; general && s0 < ns_run; s0 += 4) {
             GroupDraws<T, D, IMP ? 1 : 0> u(uint32_t(s0 >> 2), b, jb.stream, jb.seed_lo, jb.seed_hi);
             T gf = 0, ga = 0, gmf = 0, gma = 0, gmaa = 0, gmfa = 0;
             // sample s0 + k of the bin, drawing from word column kw of the group

@@ -74,7 +74,8 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         jb.bin_base = total_bins;
         total_bins += jb.nbins;
         jb.tile_base = uint32_t(total_tiles);
-        total_tiles += (jb.nbins + 255) / 256;
+        jb.tiled = vmx::bins_tiled<T>(jb.db, jb.res) ? 1 : 0;
+        total_tiles += vmx::bins_tiles<T>(jb.db, jb.res, jb.nbins);
         jb.tile_base2 = uint32_t(total_tiles2);
         total_tiles2 += vmx::rm_tiles(jb.db, jb.res, jb.nbins);
         jb.spp = p.spp;
@@ -807,7 +808,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     const double ms_str = ms_since(t_str);
 
     // ---------------- 4. bins
-    // one lane per bin, one block per tile of 256 consecutive bins of one job
+    // one lane per bin, one block per tile of 256 bins of one job
     const unsigned bins_grid = unsigned(total_tiles);  // every job starts a fresh tile
     HIP_CHECK(hipEventRecord(ctx->ev[0], st));
     const int db = jobs[0].db;
