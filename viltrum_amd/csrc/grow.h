@@ -357,18 +357,6 @@ struct Child {
     }
 };
 
-/* Appends one entry per lane with `want` to a list whose length is *n; returns the
-   lane's position.  Whole waves call it. */
-__device__ inline uint32_t wave_append(bool want, uint32_t* n) {
-    const uint64_t m = __ballot(want);
-    if (m == 0) return 0;
-    const int lane = int(threadIdx.x & 63), leader = __ffsll((unsigned long long)m) - 1;
-    int base = 0;
-    if (lane == leader) base = int(atomicAdd(n, uint32_t(__popcll(m))));
-    base = __builtin_amdgcn_readlane(base, leader);
-    return uint32_t(base) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
-}
-
 /* Inclusive sum over the lanes of a wave below and at this one, and over 16 lanes. */
 template <int CTRL, int ROWS>
 __device__ inline uint32_t dpp_add(uint32_t v) {

@@ -107,6 +107,18 @@ __device__ inline void suffix_sum256(uint32_t* s) {
     __syncthreads();
 }
 
+/* Appends one entry per lane with `want` to a list whose length is *n; returns the
+   lane's position.  Whole waves call it. */
+__device__ inline uint32_t wave_append(bool want, uint32_t* n) {
+    const uint64_t m = __ballot(want);
+    if (m == 0) return 0;
+    const int lane = int(threadIdx.x & 63), leader = __ffsll((unsigned long long)m) - 1;
+    int base = 0;
+    if (lane == leader) base = int(atomicAdd(n, uint32_t(__popcll(m))));
+    base = __builtin_amdgcn_readlane(base, leader);
+    return uint32_t(base) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+}
+
 /* pre[0] = 0, pre[j + 1] = pre[j] + count(j) for j < J, in LDS; every thread of the
    block calls it (blocks of 64..1024 threads).  Each thread sums a run of consecutive
    jobs, a shuffle scan and one exchange of the wave totals give the runs' offsets. */
@@ -375,7 +387,7 @@ __global__ void __launch_bounds__(256) k_roots(const Job<T>* __restrict__ jobs, 
     for (int idx = tid; idx < K; idx += blockDim.x) {
         T x[D];
         for (int d = 0; d < D; ++d) x[d] = node_coord<T>(double(digit3(idx, d)) / 2.0, L.box[0][0][d], L.box[0][1][d]);
-        const T y = f.template eval<M, D>(x);
+        const T y = f.template eval<Ahead<M>, D>(x);
         L.cv[0][idx] = y;
         t.v[s * K + idx] = y;
     }
@@ -743,7 +755,7 @@ __device__ inline void team_expand(const GenArgs<T>& g, const F* __restrict__ fs
     const int heur = go ? g.jobs[L.job].heur : 0;
     T e = 0;
     int dm = 0;
-    team_children<T, D, F, M>(L, t.v, fs + (go ? L.job : 0), heur, lane, go, size_t(L.slot), e, dm);
+    team_children<T, D, F, Ahead<M>>(L, t.v, fs + (go ? L.job : 0), heur, lane, go, size_t(L.slot), e, dm);
     if constexpr (LEARN) {
         // learned priority of both children (lane c scores child c); the heuristic's
         // split dim is kept, and its error stands in where the network output is NaN
@@ -884,34 +896,60 @@ __global__ void __launch_bounds__(THETA_THREADS) k_theta_round(GenArgs<T> g, int
     }
     if (g.defer == 2) {
         // jobs of up to 32768 regions: this block sorts its own job's candidates, as
-        // k_filter_round does for larger ones (one launch less per round)
+        // k_filter_round does for larger ones (one launch less per round).  Each lane has
+        // four candidates' loads in flight, a wave appends with one LDS atomic, and the
+        // deferred are counted in LDS: with a load chain and three atomics per candidate
+        // the block took 38 us a round for 256 integrals of up to 32768 regions, now 12.
         __shared__ uint32_t s_nexp, s_ndef;
+        __shared__ uint32_t s_hist[CHIST];
+        for (int i = threadIdx.x; i < CHIST; i += blockDim.x) s_hist[i] = 0;
         if (threadIdx.x == 0) {
             s_nexp = 0;
             s_ndef = 0;
         }
         __syncthreads();  // also orders the candidate histogram's clearing before its counts
-        const uint32_t nc = g.ncand[par * J + j], cs = g.cstart[par * J + j];
-        for (uint32_t i = threadIdx.x; i < ncand; i += blockDim.x) {
-            uint32_t slot;
-            T b;
-            if (i < nc) {  // a child of the last round (split already if a deepened pass took it)
-                slot = cs + i;
-                if (g.t.child[slot] >= 0) continue;
-                b = g.t.b[slot];
-            } else {
-                const DefEnt<T> e = g.def[size_t(par) * g.cap_total + jb.node_base + (i - nc)];
-                slot = e.slot;
-                b = e.b;
+        constexpr int AHEAD = 4;
+        const uint32_t nc = g.ncand[par * J + j], cs = g.cstart[par * J + j], step = blockDim.x;
+        const DefEnt<T>* from = g.def + size_t(par) * g.cap_total + jb.node_base;
+        DefEnt<T>* to = g.def + size_t(par ^ 1) * g.cap_total + jb.node_base;
+        for (uint32_t i0 = 0; i0 < ncand; i0 += AHEAD * step) {  // block-uniform
+            uint32_t slot[AHEAD];
+            T b[AHEAD];
+            int32_t child[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                const uint32_t i = i0 + uint32_t(u) * step + threadIdx.x;
+                slot[u] = NONE;
+                b[u] = T(0);
+                child[u] = -1;
+                if (i < nc) {  // a child of the last round (split already if a deepened pass took it)
+                    slot[u] = cs + i;
+                    child[u] = g.t.child[slot[u]];
+                    b[u] = g.t.b[slot[u]];
+                } else if (i < ncand) {
+                    const DefEnt<T> e = from[i - nc];
+                    slot[u] = e.slot;
+                    b[u] = e.b;
+                }
             }
-            if (b >= eff) {
-                g.exp[jb.node_base + atomicAdd(&s_nexp, 1u)] = slot;
-            } else if (b >= th) {
-                g.def[size_t(par ^ 1) * g.cap_total + jb.node_base + atomicAdd(&s_ndef, 1u)] = DefEnt<T>{slot, b};
-                atomicAdd(&g.chist[(size_t(par ^ 1) * J + j) * CHIST + (key16(b) >> 4)], 1u);
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                if (i0 + uint32_t(u) * step >= ncand) break;  // block-uniform
+                const bool open = slot[u] != NONE && child[u] < 0;
+                const bool split = open && b[u] >= eff, wait = open && !split && b[u] >= th;
+                const uint32_t at = wave_append(split, &s_nexp);
+                if (split) g.exp[jb.node_base + at] = slot[u];
+                const uint32_t k = wave_append(wait, &s_ndef);
+                if (wait) {
+                    to[k] = DefEnt<T>{slot[u], b[u]};
+                    atomicAdd(&s_hist[key16(b[u]) >> 4], 1u);
+                }
             }
         }
         __syncthreads();
+        uint32_t* next = g.chist + (size_t(par ^ 1) * J + j) * CHIST;
+        for (int i = threadIdx.x; i < CHIST; i += blockDim.x)
+            if (s_hist[i]) next[i] = s_hist[i];  // cleared above by this block, filled by the expansions later
         if (threadIdx.x == 0) {
             g.nexp[j] = s_nexp;
             g.ndef[(par ^ 1) * J + j] = s_ndef;
