@@ -2287,7 +2287,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
         // integrals of 512 x 512 bins and 4096 regions at 16 spp 1608 -> 1232 us with the
         // tiles of 16 x 16 bins, one such integral 64 -> 52 us.
         bool general = true;
-        if constexpr (FP32 && MODE == 0 && !STRAT && D <= 2) {
+        if constexpr (FP32 && !RRI && !STRAT && D <= 2) {
             if (__all((n == 1 && nf == 1) || ns_run == 0)) {
                 general = false;
                 const T* rec = r.samp + size_t(ns_run > 0 ? first0 : 0u) * SR;
@@ -2304,29 +2304,54 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
                 }
 #pragma unroll
                 for (int k = 0; k < K; ++k) coef[k] = rec[3 * D + k];
-                const T vol = box_volume<T, D>(ilo, ihi);
-                const T w = wn * vol;
+                const T box_vol = box_volume<T, D>(ilo, ihi);
                 const bool alpha1 = jb.form == VMX_FORM_CV_ALPHA1;
-                const double a1v = a1w * double(vol);
+                // Importance sampling (the rule of the general loop below): what the draws
+                // from one box share is formed once.  With the root by Newton's method
+                // (importance.h) 64 integrals of 256 x 256 bins and 4096 regions at 16 spp
+                // take 1.60 ms here, 3.61 ms with all of it per sample and root formulas
+                [[maybe_unused]] const bool srr = form_sampling_rr(jb.form);
+                [[maybe_unused]] bool drawn = false;
+                [[maybe_unused]] std::conditional_t<IMP, imp::Box<T, D>, int> pdf;
+                [[maybe_unused]] T rh[D];
+                if constexpr (IMP) {
+                    drawn = imp_form && !empty && ns_run > 0 && (srr || box_vol >= T(1.e-5));
+                    if (drawn) {
+#pragma unroll
+                        for (int d = 0; d < D; ++d) rh[d] = rec[D + d];
+                        pdf.prepare(r.v + size_t(first0) * K, rl, rh, r.vol[first0], ilo, ihi);
+                    }
+                }
                 for (uint64_t s0 = 0; s0 < ns_run; s0 += 4) {
-                    GroupDraws<T, D> u(uint32_t(s0 >> 2), b, jb.stream, jb.seed_lo, jb.seed_hi);
+                    GroupDraws<T, D, IMP ? 1 : 0> u(uint32_t(s0 >> 2), b, jb.stream, jb.seed_lo, jb.seed_hi);
                     const uint64_t left = ns_run - s0;
                     T gf = 0, ga = 0, gmf = 0, gma = 0, gmaa = 0, gmfa = 0;
+                    auto sample = [&](int k, int kw) {
+                        if (uint64_t(k) >= left) return;
+                        T x[D], t[D], vol = box_vol;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        if (uint64_t(k) >= left) break;
-                        T x[D], t[D];
+                        for (int d = 0; d < D; ++d) x[d] = mul_add<true>(u.coord(kw, d), ext[d], ilo[d]);
+                        if constexpr (IMP) {
+                            if (drawn) {
+                                T s01[D], xi[D], wgt;
 #pragma unroll
-                        for (int d = 0; d < D; ++d) {
-                            x[d] = mul_add<true>(u.coord(k, d), ext[d], ilo[d]);
-                            t[d] = (x[d] - rl[d]) * inv[d];
+                                for (int d = 0; d < D; ++d) s01[d] = u.coord(kw, d);
+                                if (pdf.draw(rl, rh, ilo, ihi, s01, xi, wgt, srr, u01f(u.extra_word(kw, 0)), vol)) {
+#pragma unroll
+                                    for (int d = 0; d < D; ++d) x[d] = xi[d];
+                                    vol = wgt;
+                                }
+                            }
                         }
+#pragma unroll
+                        for (int d = 0; d < D; ++d) t[d] = (x[d] - rl[d]) * inv[d];
                         const T fx = residual_eval<M, D>(f_lds, x);
                         const T px = eval_monomials<T, D, true>(coef, t);
                         if (alpha1) {
-                            if (!empty) acc1 += double(fx - px) * a1v;
-                            continue;
+                            if (!empty) acc1 += double(fx - px) * (a1w * double(vol));
+                            return;
                         }
+                        const T w = wn * vol;
                         const T fsv = fx * w, asv = px * w;
                         if (k == 0 && s0 == 0) {  // the bin's first sample shifts the moments
                             k_f = vabs(fsv);
@@ -2339,6 +2364,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((MODE 
                         gma += da;
                         gmaa += da * da;
                         gmfa += df * da;
+                    };
+                    if constexpr (IMP) {
+#pragma unroll 1
+                        for (int k = 0; k < 4; ++k) {
+                            sample(k, 0);
+                            u.shift();
+                        }
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) sample(k, k);
                     }
                     if (alpha1) continue;
                     sf.add(gf);
