@@ -35,10 +35,10 @@ PEAK_FP32_TFLOPS = 157.3  # MI355X published FP32 peak
 # WRITE_SIZE x1.0: the factors a 256 MiB device copy needs to read its known size), at
 # the profiled point of each workload; the commands and raw counts are in the profiles
 # named in TRAFFIC_SOURCE
-TRAFFIC_BYTES = {"config4": (131929 * 2.0 + 69097) * 1024, "config2": (8274 * 2.0 + 3072) * 1024}
+TRAFFIC_BYTES = {"config4": (232686 * 2.0 + 74303) * 1024, "config2": (8274 * 2.0 + 3072) * 1024}
 TRAFFIC_SOURCE = {
-    "config4": "PMC FETCH_SIZE/WRITE_SIZE of k_bins1 at this line's point (4096 regions, 16 spp) with the network "
-               "this bench trains (profiles/k_bins1_config4_learned_batched.md)",
+    "config4": "PMC FETCH_SIZE/WRITE_SIZE of k_bins1 at this line's point (4096 regions, 16 spp) with a learned "
+               "network (profiles/kernel_times_by_workload.md)",
     "config2": "PMC FETCH_SIZE/WRITE_SIZE of k_bins1 at 16384 regions, 64 spp (profiles/k_bins1_config2_plain.md)",
 }
 PEAK_HBM_GBS = 8000.0
