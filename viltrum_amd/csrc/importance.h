@@ -270,7 +270,7 @@ struct Box {
         at0 = cdf3(an[0], q);
         at1 = cdf3(bn[0], q);
     }
-    /* sample_regs below, of this box */
+    /* a point of the box and its weight, as described at sample_regs below */
     VMX_HD bool draw(const T* rlo, const T* rhi, const T* slo, const T* shi, const T* s, T* x, T& weight,
                      bool strategy_rr, T rr, T svol) const {
         if (strategy_rr && !(rr < den / (den + svol))) {  // the roulette chose uniform sampling
@@ -305,8 +305,8 @@ struct Box {
 };
 
 /* A point of the box [slo, shi] inside region [rlo, rhi] (volume rvol, node values v,
-   dim 0 fastest) from the uniforms s[D], and its weight (dims 1..3: the tensors in
-   registers).
+   dim 0 fastest) from the uniforms s[D], and its weight (3 dims: the tensors in
+   registers; Box draws the same in one and two).
    - strategy_rr false (region_sampling_importance, src/control-variates/
      region-sampling.h:22-44): drawn from the polynomial's pdf, weight 1/pdf (0 where
      pdf < 1e-5).  Returns false where the pdf's integral over the box is not positive
@@ -319,12 +319,7 @@ struct Box {
 template <typename T, int D>
 VMX_HD inline bool sample_regs(const T* v, const T* rlo, const T* rhi, T rvol, const T* slo, const T* shi, const T* s,
                                T* x, T& weight, bool strategy_rr, T rr, T svol) {
-    static_assert(D >= 1 && D <= 3, "register tensors: 1..3 dims");
-    if constexpr (D <= 2) {
-        Box<T, D> box;
-        box.prepare(v, rlo, rhi, rvol, slo, shi);
-        return box.draw(rlo, rhi, slo, shi, s, x, weight, strategy_rr, rr, svol);
-    }
+    static_assert(D == 3, "register tensors; Box for fewer dims, sample_deep for more");
     constexpr int K = pow3(D);
     T an[D], bn[D], un[D], pn[D];
 #pragma unroll
@@ -483,13 +478,17 @@ __attribute__((noinline)) VMX_HD bool sample_deep(const T* v, const T* rlo, cons
     return true;
 }
 
-/* A point of the box and its weight (sample_regs above for dims 1..3, sample_deep for
-   4..6); arguments and results as described at sample_regs. */
+/* A point of the box and its weight (Box above for one and two dims, sample_regs for three,
+   sample_deep for 4..6); arguments and results as described at sample_regs. */
 template <typename T, int D>
 VMX_HD inline bool sample(const T* v, const T* rlo, const T* rhi, T rvol, const T* slo, const T* shi, const T* s, T* x,
                           T& weight, bool strategy_rr = false, T rr = T(0), T svol = T(0)) {
     static_assert(D >= 1 && D <= MAX_DIM, "importance sampling: 1..6 dims");
-    if constexpr (D <= 3)
+    if constexpr (D <= 2) {
+        Box<T, D> box;
+        box.prepare(v, rlo, rhi, rvol, slo, shi);
+        return box.draw(rlo, rhi, slo, shi, s, x, weight, strategy_rr, rr, svol);
+    } else if constexpr (D == 3)
         return sample_regs<T, D>(v, rlo, rhi, rvol, slo, shi, s, x, weight, strategy_rr, rr, svol);
     else
         return sample_deep<T, D>(v, rlo, rhi, rvol, slo, shi, s, x, weight, strategy_rr, rr, svol);
