@@ -160,7 +160,8 @@ typedef struct vmx_problem {
 typedef struct vmx_stats {
     uint64_t regions;          /* final regions */
     uint64_t nodes;            /* tree nodes evaluated (>= 2*regions - 1, speculative rounds) */
-    uint64_t rounds;           /* parallel refinement rounds */
+    uint64_t rounds;           /* refinement steps: parallel rounds and one-workgroup steps
+                                  (vmx_last_generation tells them apart) */
     uint64_t pairs;            /* (bin, footprint) pairs of the per-bin lists */
     uint64_t footprints;       /* distinct bin-plane footprints */
     uint64_t evals_regions;    /* integrand evaluations for region nodes */
@@ -224,6 +225,20 @@ int vmx_integrate_regions(vmx_ctx* ctx, const vmx_problem* p, const vmx_integran
    Pass NULL arrays to query *n.  lo/hi: n*D, nodes: n*3^D, err: n, dim: n. */
 int vmx_export_regions(vmx_ctx* ctx, uint64_t* n, double* lo, double* hi, double* nodes, double* err,
                        int32_t* dim);
+
+/* How the last vmx_integrate* call on this context generated its regions, summed over
+   its groups of integrals (vmx_integrate_batch forms one per family and dimension).
+   Small integrals are generated by one workgroup each (workgroup_steps > 0, no rounds),
+   larger ones by parallel rounds of the whole chip; a larger one alone may start in a
+   workgroup (both).  The regions are the same whichever way.  All zeros where the
+   regions were given. */
+typedef struct vmx_generation {
+    uint64_t workgroup_steps; /* of the integral with the most steps */
+    uint64_t rounds;          /* parallel rounds that split regions */
+    uint64_t handovers;       /* groups that the workgroups could not finish: generated again by rounds */
+} vmx_generation;
+
+int vmx_last_generation(vmx_ctx* ctx, vmx_generation* out);
 
 /* Plain per-bin Monte Carlo with p->spp samples per bin (p->scalar, p->seed, range,
    bin_dims, res; region fields ignored): bins = volume * mean f over the bin's box.

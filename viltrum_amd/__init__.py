@@ -50,7 +50,7 @@ SYMBOLS = ["vmx_ctx_create", "vmx_ctx_destroy", "vmx_last_error", "vmx_integrate
            "vmx_integrate_batch", "vmx_export_regions", "vmx_integrate_mc", "vmx_eval", "vmx_refiner_size",
            "vmx_refiner_pairs", "vmx_refiner_train", "vmx_refiner_get", "vmx_refiner_set", "vmx_refiner_forward",
            "vmx_refiner_grad", "vmx_exact_bins", "vmx_autotune", "vmx_integrate_regions",
-           "vmx_integrate_device_noalloc"]
+           "vmx_integrate_device_noalloc", "vmx_last_generation"]
 
 
 class VmxError(RuntimeError):
@@ -73,6 +73,13 @@ class Stats(C.Structure):
         ("ties_unresolved", C.c_uint64), ("ms_generate", C.c_double), ("ms_select", C.c_double),
         ("ms_stratify", C.c_double), ("ms_bins", C.c_double), ("ms_total", C.c_double),
     ]
+
+    def as_dict(self):
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
+class Generation(C.Structure):
+    _fields_ = [("workgroup_steps", C.c_uint64), ("rounds", C.c_uint64), ("handovers", C.c_uint64)]
 
     def as_dict(self):
         return {k: getattr(self, k) for k, _ in self._fields_}
@@ -126,6 +133,7 @@ def lib():
                                           C.c_void_p]
         L.vmx_autotune.argtypes = [C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                    C.POINTER(TuneReport)]
+        L.vmx_last_generation.argtypes = [C.c_void_p, C.POINTER(Generation)]
         L.vmx_export_regions.argtypes = [C.c_void_p, C.POINTER(C.c_uint64), C.c_void_p, C.c_void_p, C.c_void_p,
                                          C.c_void_p, C.c_void_p]
         L.vmx_integrate_regions.argtypes = [C.c_void_p, C.POINTER(Problem), C.c_void_p, C.c_uint64, C.c_void_p,
@@ -252,6 +260,13 @@ class Context:
                                          hi.ctypes.data_as(C.c_void_p), nodes.ctypes.data_as(C.c_void_p),
                                          err.ctypes.data_as(C.c_void_p), dim.ctypes.data_as(C.c_void_p)))
         return dict(lo=lo, hi=hi, nodes=nodes, err=err, dim=dim)
+
+    def last_generation(self):
+        """How the last integrate call generated its regions: steps of one workgroup per
+        integral, parallel rounds, handovers from the one to the other."""
+        g = Generation()
+        self._check(lib().vmx_last_generation(self.ptr, C.byref(g)))
+        return g.as_dict()
 
     def integrate_mc(self, f, res, spp, seed, rng=None, dtype=np.float64, stratified=True):
         """Plain per-bin Monte Carlo (monte_carlo_per_bin); returns (bins, stderr)."""

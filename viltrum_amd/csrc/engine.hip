@@ -93,6 +93,7 @@ int integrate_groups(vmx_ctx* ctx, uint32_t n, const vmx_problem* const* ps, con
                      void* const* bins, vmx_stats* const* stats, hipStream_t st,
                      const GivenRegions* const* given = nullptr) {
     const int scalar = ps[0]->scalar;
+    ctx->generated = vmx_generation{};
     std::vector<int> done(n, 0);
     for (uint32_t i = 0; i < n; ++i) {
         if (ps[i]->scalar != scalar) throw VmxError(VMX_ERR_INVALID, "one scalar type per batch");
@@ -981,6 +982,14 @@ int vmx_integrate_regions(vmx_ctx* ctx, const vmx_problem* p, const vmx_integran
         HIP_CHECK(hipMemcpyAsync(bins, d, bytes, hipMemcpyDeviceToHost, ctx->stream));
         HIP_CHECK(hipStreamSynchronize(ctx->stream));
         return rc;
+    });
+}
+
+int vmx_last_generation(vmx_ctx* ctx, vmx_generation* out) {
+    return guarded(ctx, [&]() -> int {
+        if (!out) throw VmxError(VMX_ERR_INVALID, "null argument");
+        *out = ctx->generated;
+        return VMX_OK;
     });
 }
 

@@ -81,6 +81,7 @@ struct vmx_ctx {
     std::map<std::array<uint64_t, 7>, bool> grow_off;
     const Shape* trial = nullptr;
     std::vector<std::array<uint64_t, 6>> tuned_keys;
+    vmx_generation generated{};  // of the last call (vmx_last_generation)
     // last result (for vmx_export_regions): gathered from device memory on demand
     int last_D = 0;
     uint64_t last_n = 0;

@@ -155,7 +155,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     const uint32_t gen_blocks = uint32_t(n_cu) * uint32_t(shape.gen_per_cu);
     const int round_chunk = shape.round_chunk;
 
-    uint32_t rounds = 0;
+    uint32_t rounds = 0, grow_steps = 0;
     // the round-count hint's class: the workload class and the largest budget's octave
     uint32_t n_max = 1;
     for (const auto& jb : jobs) n_max = std::max(n_max, jb.N);
@@ -454,7 +454,8 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         std::memcpy(rt.data(), slot(k) + sizeof(uint32_t) * 2 * J, sizeof(vmx::JobRt) * J);
         uint32_t small_h[16];
         std::memcpy(small_h, slot(k) + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, 64);
-        rounds = small_h[0] + small_h[1];
+        rounds = small_h[0];
+        grow_steps = small_h[1];
         for (int d = 0; d < D; ++d) max_depth[d] = small_h[8 + d];
         bool cap_fail = false, too_deep = false;
         for (const auto& r : rt) {
@@ -735,9 +736,11 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         std::memcpy(rt.data(), pin + sizeof(uint32_t) * 2 * J, sizeof(vmx::JobRt) * J);
         if (grow_all) {
             std::memcpy(w, pin + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, 2 * sizeof(uint32_t));
-            rounds = w[1];
+            grow_steps = w[1];
         }
     }
+    ctx->generated.rounds += rounds;
+    ctx->generated.workgroup_steps += grow_steps;
     if (grow_all) {
         bool cap_fail = false, handed = false;
         for (const auto& r : rt) {
@@ -753,6 +756,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             } else {
                 ctx->grow_off[hint_key] = true;
             }
+            ++ctx->generated.handovers;
             if (ctx->noalloc) reset_fixed(ctx);
             return run_batch<T, D, P, Math>(ctx, in, st, pairs_req);
         }
@@ -920,7 +924,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         const auto& jb = jobs[j];
         s->regions = jb.N;
         s->nodes = rt[j].count - jb.node_base;
-        s->rounds = rounds;
+        s->rounds = rounds + grow_steps;
         s->pairs = pairs;
         s->footprints = nfp;
         s->evals_regions = uint64_t(K) + (s->nodes - 1) * uint64_t(vmx::pow3(D - 1));
