@@ -1,0 +1,90 @@
+"""Integrals that one workgroup cannot finish (its pool full of tied errors, its share of
+the tree used up) go to the parallel rounds, which generate them or refuse them: regions
+and bins bit for bit those of the rounds alone (VMX_DEFER=0), and nothing that later calls
+of the class depend on is changed by it."""
+import numpy as np
+import pytest
+
+import viltrum_amd as V
+from viltrum_amd import hip
+from viltrum_amd import integrands as I
+
+pytestmark = pytest.mark.gpu
+
+CONST = I.poly([(0.7, (0, 0))], 2)  # every region of a size ties
+POLY2 = I.poly([(1.0, (1, 2)), (0.5, (3, 0)), (0.25, (0, 0))], 2, step=([1, 1], 1.1, 0.5))
+
+
+@pytest.fixture
+def fresh():
+    c = V.Context(0)
+    yield c
+    c.close()
+
+
+def _noalloc(ctx, f, integ, res):
+    buf = hip.DeviceBuffer(4 * int(np.prod(res)))
+    try:
+        buf.zero()
+        ctx.integrate_device_noalloc(integ.problem(f, res, V.range_primary(2), V.F32), f, buf.address)
+        return buf.to_host(np.zeros(res, dtype=np.float32))
+    finally:
+        buf.free()
+
+
+def _bins(ctx, f, integ, res, dt=np.float32):
+    b = np.zeros(res, dtype=dt)
+    V.integrate(integ, b, f, V.range_primary(f.dim), ctx=ctx)
+    return b
+
+
+def test_a_refused_call_leaves_later_calls_their_memory(fresh):
+    """Every FP32 error of a constant is 0 under the absolute heuristic, so no threshold
+    ends the refinement and the call is refused whatever its budget.  16384 regions at 64
+    nodes each would not fit the no-alloc scratch; at 8 they do."""
+    res, small, large = (512, 512), V.Integrator(19, 2, 3, heuristic=V.HEUR_DEFAULT_ABSOLUTE), V.Integrator(16383, 2, 3)
+    want = _noalloc(fresh, POLY2, large, res)
+    with pytest.raises(V.VmxError, match="node capacity"):
+        _bins(fresh, CONST, small, res)
+    assert np.array_equal(_noalloc(fresh, POLY2, large, res), want)
+    assert np.array_equal(_bins(fresh, POLY2, large, res), want)
+
+
+@pytest.mark.parametrize("n", [4500, 6144])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_a_full_pool_is_generated_by_rounds(fresh, monkeypatch, n, dt):
+    integ = V.Integrator(n - 1, 2, 5)
+    got = _bins(fresh, CONST, integ, (40, 24), dt)
+    regions = fresh.export_regions(2)
+    g = fresh.last_generation()
+    assert g["handovers"] == 1 and g["workgroup_steps"] > 0 and g["rounds"] > 0
+    monkeypatch.setenv("VMX_DEFER", "0")
+    assert np.array_equal(_bins(fresh, CONST, integ, (40, 24), dt), got)
+    assert fresh.last_generation()["handovers"] == 0
+    for k, v in fresh.export_regions(2).items():
+        assert np.array_equal(v, regions[k]), k
+
+
+def test_a_full_pool_in_a_batch_and_without_allocation(fresh, monkeypatch):
+    integ = V.Integrator(4499, 2, 5)
+    got = _noalloc(fresh, CONST, integ, (40, 24))
+    assert fresh.last_generation()["handovers"] == 1
+    assert np.array_equal(_bins(fresh, CONST, integ, (40, 24)), got)
+    fs, its = [POLY2, CONST, POLY2], [V.Integrator(n - 1, 2, 7 + n) for n in (300, 4500, 1200)]
+    out = []
+    ctx = V.Context(0)
+    try:
+        for rounds in (False, True):
+            if rounds:
+                monkeypatch.setenv("VMX_DEFER", "0")
+            bufs = [hip.DeviceBuffer(4 * 40 * 24) for _ in fs]
+            ctx.integrate_batch([it.problem(f, (40, 24), V.range_primary(2), V.F32) for f, it in zip(fs, its)], fs,
+                                [b.address for b in bufs])
+            assert ctx.last_generation()["handovers"] == (0 if rounds else 1)
+            out.append([b.to_host(np.zeros((40, 24), dtype=np.float32)) for b in bufs])
+            for b in bufs:
+                b.free()
+    finally:
+        ctx.close()
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)

@@ -313,9 +313,13 @@ void launch_grow(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int32_t* le
         vmx::k_grow<T, D, P, Math, false><<<g.J, vmx::GROW_THREADS, 0, st>>>(g, d_f, leaf, select);
 }
 
-/* One (scalar, D, family) batch through the device pipeline (pipeline.h). */
+using Instant = std::chrono::steady_clock::time_point;
+
+/* One (scalar, D, family) batch through the device pipeline (pipeline.h).  left: the
+   batch's start, where k_grow's workgroups have left it to the round kernels. */
 template <typename T, int D, typename P, typename Math>
-int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsReq* pairs_req = nullptr);
+int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsReq* pairs_req = nullptr,
+              const Instant* left = nullptr);
 
 }  // namespace vmxe
 

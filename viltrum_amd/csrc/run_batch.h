@@ -24,9 +24,9 @@
 namespace vmxe {
 
 template <typename T, int D, typename P, typename Math>
-int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsReq* pairs_req) {
+int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsReq* pairs_req, const Instant* left) {
     constexpr int K = vmx::pow3(D);
-    const auto t_start = std::chrono::steady_clock::now();
+    const auto t_start = left ? *left : std::chrono::steady_clock::now();
     const uint32_t J = uint32_t(in.size());
     if (J == 0) return VMX_OK;
     if (J > uint32_t(vmx::MAX_JOBS)) throw VmxError(VMX_ERR_INVALID, "at most 4096 integrals per batch");
@@ -174,7 +174,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     // hands over once its pool fills the chip's first workgroups.  The reference's order
     // replays a heap over the rounds' nodes.  VMX_DEFER chooses among forms of the rounds,
     // so every call with it set runs them.
-    bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !std::getenv("VMX_DEFER");
+    bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !left && !std::getenv("VMX_DEFER");
     bool grow_start = grow_all && J == 1;
     if (grow_all) {
         double grow_us = 0, rounds_us = 0, splits = 0;
@@ -742,23 +742,17 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     ctx->generated.rounds += rounds;
     ctx->generated.workgroup_steps += grow_steps;
     if (grow_all) {
-        bool cap_fail = false, handed = false;
-        for (const auto& r : rt) {
-            if (r.flags & vmx::JF_DEPTH) throw VmxError(VMX_ERR_CAPACITY, "region tree deeper than 31 splits in one dim");
-            cap_fail |= (r.flags & vmx::JF_CAPACITY) != 0;
-            handed |= (r.flags & vmx::JF_HANDOVER) != 0;
-        }
-        if (cap_fail || handed) {
-            // once more, with more room or in the round kernels; nothing is in flight
-            if (cap_fail) {
-                if (cap_mult >= 64) throw VmxError(VMX_ERR_CAPACITY, "node capacity exceeded");
-                ctx->cap_hint[tune_key] = 2 * cap_mult;
-            } else {
-                ctx->grow_off[hint_key] = true;
-            }
+        uint32_t flags = 0;
+        for (const auto& r : rt) flags |= r.flags;
+        if (flags & (vmx::JF_HANDOVER | vmx::JF_CAPACITY | vmx::JF_DEPTH)) {
+            // a workgroup's pool or its integral's share of the tree is full, or a split too
+            // deep: the rounds generate the call or refuse it, with the room that the class
+            // had, so that what is refused and what a later call reserves are theirs alone;
+            // nothing is in flight
+            ctx->grow_off[hint_key] = true;
             ++ctx->generated.handovers;
             if (ctx->noalloc) reset_fixed(ctx);
-            return run_batch<T, D, P, Math>(ctx, in, st, pairs_req);
+            return run_batch<T, D, P, Math>(ctx, in, st, pairs_req, &t_start);
         }
     }
     check_pair_total(pairs64);
@@ -944,6 +938,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
 
 /* explicit instantiation of one (scalar, D, family, math policy) pipeline */
 #define VMX_INSTANTIATE_BATCH(T, D, P, M) \
-    template int vmxe::run_batch<T, D, P, M>(vmx_ctx*, const std::vector<vmxe::JobIn>&, hipStream_t, vmxe::PairsReq*);
+    template int vmxe::run_batch<T, D, P, M>(vmx_ctx*, const std::vector<vmxe::JobIn>&, hipStream_t, vmxe::PairsReq*, \
+                                             const vmxe::Instant*);
 
 #endif
