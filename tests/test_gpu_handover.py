@@ -88,3 +88,23 @@ def test_a_full_pool_in_a_batch_and_without_allocation(fresh, monkeypatch):
         ctx.close()
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+def test_one_handover_does_not_set_the_class(fresh):
+    """After a handover the next call of the class runs the rounds and the one after it
+    tries the workgroup again; while they keep failing the tries thin out."""
+    tied, plain = V.Integrator(4499, 2, 5), V.Integrator(4499, 2, 6)
+    _bins(fresh, CONST, tied, (40, 24))
+    assert fresh.last_generation()["handovers"] == 1
+    seen = []
+    for _ in range(3):
+        _bins(fresh, POLY2, plain, (40, 24))
+        g = fresh.last_generation()
+        assert g["handovers"] == 0
+        seen.append(g["rounds"] == 0)
+    assert seen == [False, True, True]
+    tries = 0
+    for _ in range(100):
+        _bins(fresh, CONST, tied, (40, 24))
+        tries += fresh.last_generation()["handovers"]
+    assert tries == 6  # at calls 1, 3, 7, 15, 31 and 63

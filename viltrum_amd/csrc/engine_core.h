@@ -77,8 +77,13 @@ struct vmx_ctx {
     // busy rounds the last call of a workload class (and budget octave) needed: where the
     // round chunks shrink
     std::map<std::array<uint64_t, 7>, uint32_t> round_hint;
-    // workload classes whose jobs did not end inside k_grow: they run the round kernels
-    std::map<std::array<uint64_t, 7>, bool> grow_off;
+    // workload classes whose last call in k_grow did not end there: their next `skip` calls
+    // run the round kernels, then one tries k_grow again (tied errors are the integrand's, so
+    // one call says little about the next); each failure in a row doubles the pause
+    struct GrowPause {
+        uint32_t skip = 0, pause = 0;
+    };
+    std::map<std::array<uint64_t, 7>, GrowPause> grow_pause;
     const Shape* trial = nullptr;
     std::vector<std::array<uint64_t, 6>> tuned_keys;
     vmx_generation generated{};  // of the last call (vmx_last_generation)

@@ -188,7 +188,14 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             grow_start &= n >= 256 && eval_us < (D <= 2 ? 10.0 : 2.0);
         }
         grow_all &= grow_us * double((J + 255) / 256) <= rounds_us + 0.0025 * splits;
-        grow_all &= order == VMX_ORDER_CANONICAL && !ctx->grow_off.count(hint_key);
+        grow_all &= order == VMX_ORDER_CANONICAL;
+        if (grow_all) {
+            const auto it = ctx->grow_pause.find(hint_key);
+            if (it != ctx->grow_pause.end() && it->second.skip > 0) {
+                --it->second.skip;
+                grow_all = false;
+            }
+        }
         for (auto& jb : jobs) jb.grow_stop = grow_all ? vmx::NONE : (D <= 2 ? 512u : 256u);
     }
     const bool grow = grow_all || grow_start;
@@ -749,11 +756,13 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             // deep: the rounds generate the call or refuse it, with the room that the class
             // had, so that what is refused and what a later call reserves are theirs alone;
             // nothing is in flight
-            ctx->grow_off[hint_key] = true;
+            auto& p = ctx->grow_pause[hint_key];
+            p.skip = p.pause = std::min(2 * p.pause + 1, 63u);
             ++ctx->generated.handovers;
             if (ctx->noalloc) reset_fixed(ctx);
             return run_batch<T, D, P, Math>(ctx, in, st, pairs_req, &t_start);
         }
+        ctx->grow_pause.erase(hint_key);
     }
     check_pair_total(pairs64);
     if (order == VMX_ORDER_CANONICAL && !replay)
