@@ -108,3 +108,17 @@ def test_one_handover_does_not_set_the_class(fresh):
         _bins(fresh, CONST, tied, (40, 24))
         tries += fresh.last_generation()["handovers"]
     assert tries == 6  # at calls 1, 3, 7, 15, 31 and 63
+
+
+# FP64 trees of 3 dims have the smallest pool, 1536 nodes
+@pytest.mark.parametrize("deepen", ["0", "1"])
+@pytest.mark.parametrize("n", [2000, 2047, 2048, 2049, 2560, 2561, 3000, 3073, 4000, 6144])
+def test_no_handover_by_size_alone(fresh, monkeypatch, n, deepen):
+    monkeypatch.setenv("VMX_DEEPEN", deepen)
+    f = I.poly([(1.0, (1, 2, 0)), (0.5, (2, 0, 1)), (0.3, (3, 1, 2))], 3, step=([1, 1, 1], 1.5, 0.25))
+    ps = [V.Integrator(n - 1, 1, i).problem(f, (6, 5), V.range_primary(3), V.F64) for i in range(64)]
+    bufs = [hip.DeviceBuffer(6 * 5 * 8) for _ in ps]
+    fresh.integrate_batch(ps, [f] * len(ps), [b.address for b in bufs])
+    for b in bufs:
+        b.free()
+    assert fresh.last_generation()["handovers"] == 0

@@ -306,6 +306,16 @@ constexpr bool grow_built(bool learn) {
     return D <= (learn ? 2 : 3);
 }
 
+/* The largest integral that k_grow is given: its measured range, and what its pool holds.
+   Until N - 1 nodes are known none is dropped, so the pool holds every unsplit node, N / 2
+   of them, and a step adds one for each split. */
+template <typename T, int D>
+constexpr uint32_t grow_limit(bool deepen) {
+    using S = vmx::GrowShape<T, D, false>;
+    const uint32_t pool = 2u * uint32_t(S::POOL - S::SPLITS * (deepen ? 2 : 1));
+    return pool < 6144u ? pool : 6144u;
+}
+
 template <typename T, int D, typename P, typename Math>
 void launch_grow(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int32_t* leaf, int select, hipStream_t st) {
     if constexpr (std::is_same<T, float>::value && grow_built<D>(true) && !vmx::IsFubini<P>::value) {

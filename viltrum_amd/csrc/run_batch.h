@@ -184,7 +184,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             grow_us = std::max(grow_us, 8.0 * (4.0 + eval_us) + (n / 256.0 + 4.0) * step_us + 10.0 + n / 100.0);
             rounds_us = std::max(rounds_us, ((learn ? 30.0 : 20.0) + eval_us) * (7.0 + std::log2(n)) + 45.0);
             splits += n;
-            grow_all &= n <= 6144;
+            grow_all &= jobs[j].N <= grow_limit<T, D>(shape.deepen != 0);
             grow_start &= n >= 256 && eval_us < (D <= 2 ? 10.0 : 2.0);
         }
         grow_all &= grow_us * double((J + 255) / 256) <= rounds_us + 0.0025 * splits;
