@@ -35,7 +35,7 @@ constexpr int GROW_WAVES = 8, GROW_THREADS = 64 * GROW_WAVES;
 constexpr int GROW_BUCKETS = 4096;
 constexpr uint32_t GROW_MAX_NODES = 65535;  // node indexes within a job are 16 bits here
 constexpr uint32_t GROW_MAX_REGIONS = 8192;
-constexpr uint32_t GROW_DIRECT = 1024;  // boundary buckets up to this are ranked directly
+constexpr uint32_t GROW_DIRECT = 256;  // boundary buckets up to this are ranked directly
 
 /* Buckets of the priorities, 32 per octave over 128 octaves up to `top`; values above
    share the last bucket, values below the first.  lower(k) is at most every value of
@@ -115,11 +115,16 @@ struct GrowLds {
         uint16_t idx[2][GROW_MAX_REGIONS];           // ping-pong of the sort; idx[1] first lists the bucket
         uint8_t state[GROW_MAX_REGIONS];             // of the bucket's nodes: 0 undecided, 1 split, 2 kept
         T b[GROW_DIRECT];                            // their b, for a direct ranking
-        uint32_t key[GROW_MAX_REGIONS];              // the sort's packed codes, and their nodes
+        uint32_t key[GROW_MAX_REGIONS];              // the sort's packed codes, and their nodes; codes of ties
         uint16_t node[GROW_MAX_REGIONS];
         uint32_t whist[S::WAVES][256];
         uint32_t digit[256];
+        // the second keys of the bucket's nodes, before the sort's lists take the memory
+        __device__ T* tie_b1() { return reinterpret_cast<T*>(&idx[0][0]); }
     };
+    static_assert(GROW_DIRECT <= GROW_THREADS, "a thread per node of the bucket");
+    static_assert(sizeof(uint16_t) * GROW_MAX_REGIONS >= sizeof(T) * GROW_DIRECT && GROW_MAX_REGIONS >= 3 * GROW_DIRECT,
+                  "second keys and codes of a bucket");
     union {
         Gen g;
         Sel s;
@@ -135,6 +140,7 @@ struct GrowLds {
     uint32_t kb, above, kt;  // theta's bucket and the nodes above it, tau's bucket
     uint32_t depth[VMX_MAX_DIM];
     uint32_t top_row, nsel, ties, dsel, dabove, dleft, flags;
+    uint32_t kor, kand;
     int32_t last;
 };
 
@@ -433,6 +439,18 @@ __device__ inline void grow_thresholds(GrowLds<T, D, LEARN>& L, uint32_t need, u
     lds_barrier();
 }
 
+/* Word w of the full key (b, b1, ~codes) of the node in slot s, the most significant first. */
+template <typename T, int D>
+__device__ inline uint32_t grow_key_word(const TreeArrays<T>& t, size_t s, int w) {
+    constexpr int W = int(sizeof(T)) / 4;
+    if (w >= 2 * W) return ~t.code[s * D + (w - 2 * W)];
+    const T v = w < W ? t.b[s] : t.b1[s];
+    if constexpr (W == 1)
+        return __float_as_uint(float(v));
+    else
+        return uint32_t(uint64_t(__double_as_longlong(double(v))) >> (w % W == 0 ? 32 : 0));
+}
+
 /* Exact selection and canonical order of a job that has grown to the end: the nodes above
    theta's bucket are split, the (need - above) largest of it too by the full key
    (b, b1, ~codes), and the unsplit children of split nodes, sorted by (code_0, ...,
@@ -475,92 +493,135 @@ __device__ inline uint32_t grow_select(GrowLds<T, D, LEARN>& L, const TreeArrays
     if (need > 0) {
         const uint32_t take = need - above;  // this many of the bucket's nodes are split
         if (nb <= GROW_DIRECT) {
-            // each node's place by counting the larger keys; b decides nearly always
-            for (uint32_t i = tid; i < nb; i += NT) L.s.b[i] = t.b[base + L.s.idx[1][i]];
+            // each node's place by counting the larger keys; b decides nearly always, and where
+            // some tie (siblings that inherit their parent's b) the rest of their keys come to
+            // LDS too
+            const uint32_t i = uint32_t(tid);
+            const bool own = i < nb;
+            const T bi = own ? t.b[base + L.s.idx[1][i]] : T(0);
+            if (own) L.s.b[i] = bi;
             __syncthreads();
-            for (uint32_t i = tid; i < nb; i += NT) {
-                const T bi = L.s.b[i];
-                uint32_t larger = 0;
-                bool tied = false;
+            uint32_t larger = 0;
+            bool tied = false;
+            for (uint32_t k = 0; k < nb; ++k) {
+                const T bk = L.s.b[k];
+                larger += bk > bi ? 1u : 0u;
+                tied |= bk == bi && k != i;
+            }
+            if (__syncthreads_or(own && tied)) {
+                T* const b1 = L.s.tie_b1();
+                uint32_t* const code = L.s.key;
+                T b1i = T(0);
+                uint32_t ci[D] = {};
+                if (own) {
+                    const size_t s = size_t(base) + L.s.idx[1][i];
+                    b1[i] = b1i = t.b1[s];
+#pragma unroll
+                    for (int d = 0; d < D; ++d) code[uint32_t(d) * GROW_DIRECT + i] = ci[d] = t.code[s * D + d];
+                }
+                __syncthreads();
                 for (uint32_t k = 0; k < nb; ++k) {
-                    const T bk = L.s.b[k];
-                    larger += bk > bi ? 1u : 0u;
-                    tied |= bk == bi && k != i;
+                    const T b1k = b1[k];
+                    bool same = true, first = false;  // smaller codes first
+#pragma unroll
+                    for (int d = 0; d < D; ++d) {
+                        const uint32_t ck = code[uint32_t(d) * GROW_DIRECT + k];
+                        first |= same && ck < ci[d];
+                        same &= ck == ci[d];
+                    }
+                    larger += L.s.b[k] == bi && (b1k > b1i || (b1k == b1i && first)) ? 1u : 0u;
                 }
-                if (tied) {
-                    const size_t si = size_t(base) + L.s.idx[1][i];
-                    for (uint32_t k = 0; k < nb; ++k)
-                        if (L.s.b[k] == bi && k != i) {
-                            const size_t sk = size_t(base) + L.s.idx[1][k];
-                            int cmp = t.b1[sk] > t.b1[si] ? 1 : (t.b1[sk] < t.b1[si] ? -1 : 0);
-                            for (int d = 0; d < D && cmp == 0; ++d) {
-                                const uint32_t ck = t.code[sk * D + d], ci = t.code[si * D + d];
-                                cmp = ck < ci ? 1 : (ck > ci ? -1 : 0);
-                            }
-                            larger += cmp > 0 ? 1u : 0u;
-                        }
-                }
+            }
+            if (own) {
                 const uint32_t x = L.s.idx[1][i];
                 L.s.state[i] = larger < take ? 1 : 2;
                 if (larger + 1 == take) L.last = int32_t(x);
                 if (larger < take) atomicOr(reinterpret_cast<unsigned long long*>(&L.s.split[x >> 6]), 1ull << (x & 63));
             }
         } else {
-        // radix selection inside the bucket, a byte per pass from the first byte the
-        // bucket does not fix, until one undecided node is left (keys are unique)
-        constexpr int BB = int(sizeof(T)), FIRST = 0, PASSES = (BB - FIRST) + BB + 4 * D;
-        auto digit_of = [&](uint32_t i, int pass) -> uint32_t {
-            const size_t s = size_t(base) + i;
-            if (pass < BB - FIRST) {
-                const int sh = 8 * (BB - 1 - FIRST - pass);
-                if constexpr (BB == 4)
-                    return (__float_as_uint(float(t.b[s])) >> sh) & 0xFFu;
-                else
-                    return uint32_t(uint64_t(__double_as_longlong(double(t.b[s]))) >> sh) & 0xFFu;
+            // radix selection over the keys' 32-bit words, a byte per pass, until one
+            // undecided node is left (keys are unique).  A thread's nodes and their current
+            // word are in registers, and bytes that all undecided nodes share are passed
+            // over: regions of a size over flat parts differ in their codes alone.  The whole
+            // kernel, for a constant (1024 tied nodes in the bucket: 2 dims, FP64, 1600 regions,
+            // and 3 dims) 727 -> 125 and 1042 -> 338 us, against buckets of up to 1024 ranked
+            // directly with the ties' keys in device memory; 2 dims, FP32, 300 regions (768
+            // nodes) 476 -> 90; a polynomial of 4000 regions 219 -> 216 (ranking costs the
+            // square of the bucket: 55 us at 1024 nodes without ties, a pass here 4)
+            constexpr int W = int(sizeof(T)) / 4, PER = int(GROW_MAX_REGIONS) / NT;
+            uint32_t x[PER], word[PER], open = 0, up = 0;  // open, up: bit per own node
+#pragma unroll
+            for (int r = 0; r < PER; ++r) {
+                const uint32_t i = uint32_t(r * NT + tid);
+                x[r] = i < nb ? uint32_t(L.s.idx[1][i]) : 0u;
+                open |= i < nb ? 1u << r : 0u;
             }
-            pass -= BB - FIRST;
-            if (pass < BB) {
-                const int sh = 8 * (BB - 1 - pass);
-                if constexpr (BB == 4)
-                    return (__float_as_uint(float(t.b1[s])) >> sh) & 0xFFu;
-                else
-                    return uint32_t(uint64_t(__double_as_longlong(double(t.b1[s]))) >> sh) & 0xFFu;
-            }
-            pass -= BB;
-            return (~t.code[s * D + pass / 4] >> (8 * (3 - pass % 4))) & 0xFFu;
-        };
-        uint32_t rank = take;
-        for (int pass = 0; pass < PASSES; ++pass) {
-            if (tid < 256) L.s.digit[tid] = 0;
-            __syncthreads();
-            for (uint32_t i = tid; i < nb; i += NT)
-                if (L.s.state[i] == 0) atomicAdd(&L.s.digit[digit_of(L.s.idx[1][i], pass)], 1u);
-            __syncthreads();
-            const uint32_t own = tid < 256 ? L.s.digit[tid] : 0u;
-            __syncthreads();
-            suffix_sum256(L.s.digit);
-            if (tid < 256 && L.s.digit[tid] >= rank && (tid == 255 || L.s.digit[tid + 1] < rank)) {
-                L.dsel = uint32_t(tid);
-                L.dabove = L.s.digit[tid] - own;
-                L.dleft = own;
-            }
-            __syncthreads();
-            const uint32_t dsel = L.dsel, left = L.dleft;
-            for (uint32_t i = tid; i < nb; i += NT)
-                if (L.s.state[i] == 0) {
-                    const uint32_t dg = digit_of(L.s.idx[1][i], pass);
-                    if (dg != dsel) L.s.state[i] = dg > dsel ? 1 : 2;
+            uint32_t rank = take, left = nb;
+            for (int w = 0; w < 2 * W + D && left > 1; ++w) {
+                if (tid == 0) {
+                    L.kor = 0;
+                    L.kand = NONE;
                 }
-            rank -= L.dabove;
-            __syncthreads();
-            if (left == 1) break;
-        }
-        for (uint32_t i = tid; i < nb; i += NT) {
-            const uint32_t x = L.s.idx[1][i];
-            if (L.s.state[i] == 0) L.last = int32_t(x);
-            if (L.s.state[i] != 2)
-                atomicOr(reinterpret_cast<unsigned long long*>(&L.s.split[x >> 6]), 1ull << (x & 63));
-        }
+                uint32_t any = 0, all = NONE;
+#pragma unroll
+                for (int r = 0; r < PER; ++r) word[r] = open >> r & 1u ? grow_key_word<T, D>(t, size_t(base) + x[r], w) : 0u;
+#pragma unroll
+                for (int r = 0; r < PER; ++r)
+                    if (open >> r & 1u) {
+                        any |= word[r];
+                        all &= word[r];
+                    }
+                for (int o = 32; o > 0; o >>= 1) {
+                    any |= uint32_t(__shfl_xor(int(any), o, 64));
+                    all &= uint32_t(__shfl_xor(int(all), o, 64));
+                }
+                __syncthreads();
+                if (lane == 0) {
+                    atomicOr(&L.kor, any);
+                    atomicAnd(&L.kand, all);
+                }
+                __syncthreads();
+                const uint32_t differ = L.kor ^ L.kand;
+                for (int sh = differ ? (31 - __clz(int(differ))) & ~7 : -1; sh >= 0 && left > 1; sh -= 8) {
+                    if ((differ >> sh & 0xFFu) == 0) continue;
+                    if (tid < 256) L.s.digit[tid] = 0;
+                    __syncthreads();
+#pragma unroll
+                    for (int r = 0; r < PER; ++r)
+                        if (open >> r & 1u) atomicAdd(&L.s.digit[word[r] >> sh & 0xFFu], 1u);
+                    __syncthreads();
+                    const uint32_t own = tid < 256 ? L.s.digit[tid] : 0u;
+                    __syncthreads();
+                    suffix_sum256(L.s.digit);
+                    if (tid < 256 && L.s.digit[tid] >= rank && (tid == 255 || L.s.digit[tid + 1] < rank)) {
+                        L.dsel = uint32_t(tid);
+                        L.dabove = L.s.digit[tid] - own;
+                        L.dleft = own;
+                    }
+                    __syncthreads();
+                    const uint32_t dsel = L.dsel;
+#pragma unroll
+                    for (int r = 0; r < PER; ++r)
+                        if (open >> r & 1u) {
+                            const uint32_t dg = word[r] >> sh & 0xFFu;
+                            if (dg != dsel) open &= ~(1u << r);
+                            if (dg > dsel) up |= 1u << r;
+                        }
+                    rank -= L.dabove;
+                    left = L.dleft;
+                    __syncthreads();
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int r = 0; r < PER; ++r) {
+                const uint32_t i = uint32_t(r * NT + tid);
+                if (i >= nb) break;
+                if (open >> r & 1u) L.last = int32_t(x[r]);
+                const bool split = (open | up) >> r & 1u;
+                L.s.state[i] = split ? 1 : 2;
+                if (split) atomicOr(reinterpret_cast<unsigned long long*>(&L.s.split[x[r] >> 6]), 1ull << (x[r] & 63));
+            }
         }
         __syncthreads();
         if (L.last >= 0) {
