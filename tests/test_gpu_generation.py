@@ -45,3 +45,32 @@ def test_groups_of_a_batch_are_summed_and_given_regions_have_none(ctx):
     V.integrate(it, b, BLOBS, V.range_primary(2), ctx=ctx)
     V.integrate_regions(it, b, BLOBS, V.range_primary(2), ctx.export_regions(2), ctx=ctx)
     assert _ways(ctx.last_generation()) == (False, False, 0)
+
+
+POLY3 = I.poly([(1.0, (1, 2, 0)), (0.5, (2, 0, 1)), (0.3, (3, 1, 2))], 3, step=([1, 1, 1], 1.5, 0.25))
+LONG3 = I.poly([(0.1 * (k + 1), (k % 4, (k + 1) % 4, (k + 2) % 3)) for k in range(12)], 3)
+MOVING8 = I.moving_blobs(3, 8)
+
+
+# both sides of the choice, at sizes where one generator was measured 10 % or more ahead
+@pytest.mark.parametrize("f,dt,jobs,n,workgroup", [
+    (POLY3, np.float64, 1, 1600, False), (MOVING8, np.float64, 1, 800, False), (POLY3, np.float32, 1, 4000, False),
+    (LONG3, np.float32, 1, 2400, False), (MOVING8, np.float32, 1, 6000, False), (POLY3, np.float64, 1, 20, True),
+    (MOVING8, np.float32, 1, 800, True), (BLOBS, np.float32, 1, 6144, True), (BLOBS, np.float64, 1, 4000, True),
+    (POLY3, np.float64, 64, 400, True), (POLY3, np.float32, 64, 2400, True)],
+    ids=lambda v: getattr(v, "__name__", str(v)) if not hasattr(v, "desc") else "f%d" % v.dim)
+def test_the_faster_generator_is_chosen(ctx, f, dt, jobs, n, workgroup):
+    res = (24, 17)
+    ps = [V.Integrator(n - 1, 1, i).problem(f, res, V.range_primary(f.dim), V.F32 if dt == np.float32 else V.F64)
+          for i in range(jobs)]
+    bufs = [hip.DeviceBuffer(24 * 17 * 8) for _ in ps]
+    ctx.integrate_batch(ps, [f] * jobs, [b.address for b in bufs])
+    for b in bufs:
+        b.free()
+    g = ctx.last_generation()
+    assert (g["rounds"] == 0) == workgroup and g["handovers"] == 0, g
+
+
+def test_starts_in_a_workgroup_where_that_gains(ctx):
+    assert _ways(_integrate(ctx, MOVING8, 20000)) == (True, True, 0)
+    assert _ways(_integrate(ctx, POLY3, 20000, dt=np.float64)) == (False, True, 0)

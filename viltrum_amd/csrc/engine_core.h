@@ -280,24 +280,54 @@ void launch_expand(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int par, 
     vmx::k_expand_round<T, D, P, Math, false><<<blocks, vmx::GEN_THREADS, pre_bytes, st>>>(g, d_f, par);
 }
 
-/* Rough instruction count of one evaluation, for the choice of how regions are generated
-   (a user's functor: a middling guess). */
+/* Rough instruction count of one evaluation in `dim` dims, for the choice of how regions
+   are generated, from k_grow's time a step (a user's functor: a middling guess). */
 template <typename P>
-double eval_work(const P&) {
+double eval_work(const P&, int) {
     return 100.0;
 }
 template <typename T>
-double eval_work(const vmx::Poly<T>& p) {
-    return 30.0 + 12.0 * p.nterms;
+double eval_work(const vmx::Poly<T>& p, int dim) {  // a loop per term and dim
+    return 30.0 + 16.0 * dim * p.nterms;
 }
 template <typename T>
-double eval_work(const vmx::Blobs<T>& p) {  // FP64: the precise exp, sin and cos
-    return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 80.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
+double eval_work(const vmx::Blobs<T>& p, int) {  // FP64: the precise exp, sin and cos
+    return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 40.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
 }
 template <typename T, typename Inner, int DF, int RD>
-double eval_work(const vmx::Fubini<T, Inner, DF, RD>& p) {
-    return double(p.mc) * (80.0 + eval_work(p.in));
+double eval_work(const vmx::Fubini<T, Inner, DF, RD>& p, int) {
+    return double(p.mc) * (80.0 + eval_work(p.in, DF));
 }
+/* ... in us on a lane: 8 cycles an instruction. */
+template <int D, typename P>
+double eval_us(const P& p) {
+    return 0.0033 * eval_work(p, D);
+}
+
+/* k_grow's time for the splits of an integral of n regions, us: a step for each 256, which
+   is issue-bound on one CU. */
+template <typename T, int D>
+double grow_us(bool learn, double n, double eval) {
+    const double step = learn ? (D == 1 ? 7.0 : 15.0) : (D <= 2 ? 7.0 : (sizeof(T) == 8 ? 27.0 : 15.0));
+    return n / 256.0 * (step + 1.3 * vmx::pow3(D - 1) * eval);
+}
+/* What the rounds and their selection cost more than k_grow without those steps, us: two
+   launches a round, a round per level, more of both with many integrals, and the chip's
+   time for the splits.  Fitted with the steps above to both generators over 2400 calls: polynomials of 1 to 12
+   terms, 1 to 64 static and 2 to 32 moving blobs, Fubini forms, learned priorities, 2 to
+   6144 regions, 1 to 300 integrals.  Where this rule takes k_grow it is at most 4 % behind
+   the rounds, but for two of those calls (7 %); where it takes the rounds they are at most
+   30 % behind, beside the line.  FP64 in 3 dims spills (a child is 27 values in a lane):
+   rounds from 100 to 300 regions on, one integral. */
+template <typename T, int D>
+double rounds_us(bool learn, double n, double jobs, double splits) {
+    const double base = learn ? 30.0 : (D == 3 && sizeof(T) == 8 ? 30.0 : 40.0);
+    const double level = learn ? (D == 1 ? 15.0 : 23.0) : (D == 1 ? 30.0 : (D == 2 ? 19.0 : (sizeof(T) == 8 ? 0.0 : 12.0)));
+    const double octave = learn ? 12.0 : (D == 1 ? 22.0 : (D == 2 ? 14.0 : 7.0));
+    const double split = D == 1 ? 0.0018 : (D == 2 ? 0.0013 : 0.0021);
+    return base + level * std::log2(n) + octave * std::log2(std::min(jobs, 64.0)) + split * splits;
+}
+constexpr double GROW_WAVE_US = 45.0;  // of each further wave of workgroups
 
 /* Whether k_grow is built for a pipeline: a child of a split in the registers of one lane
    (D <= 3), with the learned priority the network beside it in LDS (D <= 2). */

@@ -162,32 +162,28 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     std::array<uint64_t, 7> hint_key{};
     std::copy(tune_key.begin(), tune_key.end(), hint_key.begin());
     hint_key[6] = uint64_t(ilog2(n_max));
-    // One workgroup per integral generates it (grow.h) where that beats the rounds; both
-    // sides as measured (us).  k_grow: 8 steps while the tree is small, then a step for each
-    // 256 splits, issue-bound on one CU (5.5 and the 3^(D-1) evaluations of a lane; 14 for 3
-    // dims, 13 with the network), and the selection.  Rounds: about log2 N + 7 of two
-    // launches each, 20 and an evaluation (30 with the network), 2.5 ns a split, and the
-    // selection's launches.  One 2-D integral of 1024 / 2048 / 4096 regions: 370 / 400 / 500
-    // by rounds, 80 / 115 / 230 here; 64 learned ones of 4096 regions 1520 -> 430; 3 dims
-    // with 8 blobs cross over near 3000 regions, 2 dims with 64 blobs near 6000.  A larger
-    // integral alone starts here (the rounds of a handful of regions are all launch) and
-    // hands over once its pool fills the chip's first workgroups.  The reference's order
-    // replays a heap over the rounds' nodes.  VMX_DEFER chooses among forms of the rounds,
-    // so every call with it set runs them.
+    // One workgroup per integral generates it (grow.h) where that beats the rounds, both
+    // sides as measured (engine_core.h): a 2-D integral of 1024 / 2048 / 4096 regions takes
+    // 370 / 400 / 500 us by rounds, 80 / 115 / 230 here; 64 learned ones of 4096 regions
+    // 1520 -> 430; 3 dims with 8 blobs cross over near 2500 regions.  A larger integral
+    // alone starts here (the rounds of a handful of regions are all launch) and hands over
+    // once its pool fills the chip's first workgroups: 3 to 25 % of a call in 1 and 2 dims,
+    // 1 to 6 % in 3 from 400 regions (below, and where an evaluation takes 2 us, nothing;
+    // FP64 loses 8 to 30 %).  The reference's order replays a heap over the rounds' nodes.
+    // VMX_DEFER chooses among forms of the rounds, so every call with it set runs them.
     bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !left && !std::getenv("VMX_DEFER");
-    bool grow_start = grow_all && J == 1;
+    bool grow_start = grow_all && J == 1 && (D <= 2 || sizeof(T) == 4);
     if (grow_all) {
-        double grow_us = 0, rounds_us = 0, splits = 0;
+        double grow = 0, splits = 0;
         for (uint32_t j = 0; j < J; ++j) {
-            const double eval_us = 0.0033 * eval_work(fparams[j]);  // 8 cycles an instruction
-            const double n = jobs[j].N, step_us = (learn ? 13.0 : (D <= 2 ? 5.5 : 14.0)) + 1.3 * vmx::pow3(D - 1) * eval_us;
-            grow_us = std::max(grow_us, 8.0 * (4.0 + eval_us) + (n / 256.0 + 4.0) * step_us + 10.0 + n / 100.0);
-            rounds_us = std::max(rounds_us, ((learn ? 30.0 : 20.0) + eval_us) * (7.0 + std::log2(n)) + 45.0);
-            splits += n;
+            const double eval = eval_us<D>(fparams[j]);
+            grow = std::max(grow, grow_us<T, D>(learn, jobs[j].N, eval));
+            splits += jobs[j].N;
             grow_all &= jobs[j].N <= grow_limit<T, D>(shape.deepen != 0);
-            grow_start &= n >= 256 && eval_us < (D <= 2 ? 10.0 : 2.0);
+            grow_start &= D <= 2 ? jobs[j].N >= 256 && eval < 20.0 : jobs[j].N >= 400 && eval < 1.6;
         }
-        grow_all &= grow_us * double((J + 255) / 256) <= rounds_us + 0.0025 * splits;
+        const double waves = (J + uint32_t(n_cu) - 1) / uint32_t(n_cu);
+        grow_all &= grow * waves + GROW_WAVE_US * (waves - 1) <= rounds_us<T, D>(learn, n_max, J, splits);
         grow_all &= order == VMX_ORDER_CANONICAL;
         if (grow_all) {
             const auto it = ctx->grow_pause.find(hint_key);
