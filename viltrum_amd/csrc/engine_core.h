@@ -294,6 +294,12 @@ template <typename T>
 double eval_work(const vmx::Blobs<T>& p, int) {  // FP64: the precise exp, sin and cos
     return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 40.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
 }
+/* A wave runs to its longest series, log(64) / -log(decay) terms: 1, 4 and 20 us a sample at
+   decay 0.3, 0.75 and 0.95. */
+template <typename T>
+double eval_work(const vmx::Dyson<T>& p, int) {
+    return 80.0 * std::max(1.0, 4.7 / -std::log(double(p.decay)));
+}
 template <typename T, typename Inner, int DF, int RD>
 double eval_work(const vmx::Fubini<T, Inner, DF, RD>& p, int) {
     return double(p.mc) * (80.0 + eval_work(p.in, DF));

@@ -167,9 +167,9 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     // 370 / 400 / 500 us by rounds, 80 / 115 / 230 here; 64 learned ones of 4096 regions
     // 1520 -> 430; 3 dims with 8 blobs cross over near 2500 regions.  A larger integral
     // alone starts here (the rounds of a handful of regions are all launch) and hands over
-    // once its pool fills the chip's first workgroups: 3 to 25 % of a call in 1 and 2 dims,
-    // 1 to 6 % in 3 from 400 regions (below, and where an evaluation takes 2 us, nothing;
-    // FP64 loses 8 to 30 %).  The reference's order replays a heap over the rounds' nodes.
+    // once its pool fills the chip's first workgroups: 3 to 25 % of a call in 1 dim and in 2
+    // (nothing there from 15 us an evaluation, a loss from 20), 1 to 6 % in 3 from 400
+    // regions (nothing at 2 us, a loss above; FP64 loses 8 to 30 %).  The reference's order replays a heap over the rounds' nodes.
     // VMX_DEFER chooses among forms of the rounds, so every call with it set runs them.
     bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !left && !std::getenv("VMX_DEFER");
     bool grow_start = grow_all && J == 1 && (D <= 2 || sizeof(T) == 4);
@@ -180,7 +180,8 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
             grow = std::max(grow, grow_us<T, D>(learn, jobs[j].N, eval));
             splits += jobs[j].N;
             grow_all &= jobs[j].N <= grow_limit<T, D>(shape.deepen != 0);
-            grow_start &= D <= 2 ? jobs[j].N >= 256 && eval < 20.0 : jobs[j].N >= 400 && eval < 1.6;
+            grow_start &= D == 1 ? jobs[j].N >= 256
+                                 : (D == 2 ? jobs[j].N >= 256 && eval < 10.0 : jobs[j].N >= 400 && eval < 1.6);
         }
         const double waves = (J + uint32_t(n_cu) - 1) / uint32_t(n_cu);
         grow_all &= grow * waves + GROW_WAVE_US * (waves - 1) <= rounds_us<T, D>(learn, n_max, J, splits);
