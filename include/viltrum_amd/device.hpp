@@ -22,6 +22,16 @@
  * VMX_CUSTOM_MAX_BYTES: its bytes are copied to device memory per integral (captured
  * parameters travel with it, pointers in it must be device pointers).
  *
+ * A functor may state what an evaluation takes, in instructions, roughly, in a member
+ *
+ *     double evaluation_work() const { return 40; }
+ *
+ * (host code).  Small integrals in up to three dims are then generated by one workgroup
+ * each wherever that is faster: 1024 regions of a cheap functor in two dims 550 -> 260 us a
+ * call.  Without it they are generated by the chip's parallel rounds, which suit a functor
+ * of any cost: one of 30000 instructions takes 7.0 ms for 4000 regions in a workgroup, 4.0
+ * by rounds.  The results are the same.
+ *
  * The scalar types to instantiate follow the dimension argument: device_integrand<D>(f) builds
  * the FP32 path (float bins), device_integrand<D, double>(f) the FP64 path and
  * device_integrand<D, float, double>(f) both; bins of a type not instantiated are

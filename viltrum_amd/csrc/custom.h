@@ -151,6 +151,27 @@ struct F64Of<vmx::Custom<T, DIM, Fn>> {
     using type = vmx::Custom<double, DIM, Fn>;
 };
 
+/* What a functor's member `evaluation_work()` says an evaluation takes, in instructions. */
+template <typename Fn, typename = void>
+struct StatedWork {
+    static double of(const void*) { return std::numeric_limits<double>::infinity(); }
+};
+template <typename Fn>
+struct StatedWork<Fn, std::void_t<decltype(double(std::declval<const Fn&>().evaluation_work()))>> {
+    static double of(const void* raw) {
+        const double w = double(static_cast<const Fn*>(raw)->evaluation_work());
+        return w > 0 ? w : std::numeric_limits<double>::infinity();
+    }
+};
+template <typename T, int DIM, typename Fn>
+struct EvalWork<vmx::Custom<T, DIM, Fn>> {
+    static double of(const vmx::Custom<T, DIM, Fn>& p, int) { return StatedWork<Fn>::of(p.raw); }
+};
+template <typename T, typename Fn>
+struct EvalWork<vmx::CustomSeq<T, Fn>> {
+    static double of(const vmx::CustomSeq<T, Fn>& p, int) { return StatedWork<Fn>::of(p.raw); }
+};
+
 }  // namespace vmxe
 
 #endif

@@ -281,33 +281,42 @@ void launch_expand(bool learn, const vmx::GenArgs<T>& g, const P* d_f, int par, 
 }
 
 /* Rough instruction count of one evaluation in `dim` dims, for the choice of how regions
-   are generated, from k_grow's time a step (a user's functor: a middling guess). */
+   are generated, from k_grow's time a step.  Infinite where nothing is known (a user's
+   functor that does not state it): the rounds, whose time depends on it the least. */
 template <typename P>
-double eval_work(const P&, int) {
-    return 100.0;
-}
+struct EvalWork {
+    static double of(const P&, int) { return std::numeric_limits<double>::infinity(); }
+};
 template <typename T>
-double eval_work(const vmx::Poly<T>& p, int dim) {  // a loop per term and dim
-    return 30.0 + 16.0 * dim * p.nterms;
-}
+struct EvalWork<vmx::Poly<T>> {  // a loop per term and dim
+    static double of(const vmx::Poly<T>& p, int dim) { return 30.0 + 16.0 * dim * p.nterms; }
+};
 template <typename T>
-double eval_work(const vmx::Blobs<T>& p, int) {  // FP64: the precise exp, sin and cos
-    return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 40.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
-}
+struct EvalWork<vmx::Blobs<T>> {  // FP64: the precise exp, sin and cos
+    static double of(const vmx::Blobs<T>& p, int) {
+        return sizeof(T) == 8 ? 20.0 + (p.wa != 0 ? 400.0 : 0.0) + 40.0 * p.nblobs : 40.0 + 13.0 * p.nblobs;
+    }
+};
+template <typename T>
+struct EvalWork<vmx::Lobes5<T>> {
+    static double of(const vmx::Lobes5<T>&, int) { return 50.0; }
+};
 /* A wave runs to its longest series, log(64) / -log(decay) terms: 1, 4 and 20 us a sample at
    decay 0.3, 0.75 and 0.95. */
 template <typename T>
-double eval_work(const vmx::Dyson<T>& p, int) {
-    return 80.0 * std::max(1.0, 4.7 / -std::log(double(p.decay)));
-}
+struct EvalWork<vmx::Dyson<T>> {
+    static double of(const vmx::Dyson<T>& p, int) { return 80.0 * std::max(1.0, 4.7 / -std::log(double(p.decay))); }
+};
 template <typename T, typename Inner, int DF, int RD>
-double eval_work(const vmx::Fubini<T, Inner, DF, RD>& p, int) {
-    return double(p.mc) * (80.0 + eval_work(p.in, DF));
-}
+struct EvalWork<vmx::Fubini<T, Inner, DF, RD>> {
+    static double of(const vmx::Fubini<T, Inner, DF, RD>& p, int) {
+        return double(p.mc) * (80.0 + EvalWork<Inner>::of(p.in, DF));
+    }
+};
 /* ... in us on a lane: 8 cycles an instruction. */
 template <int D, typename P>
 double eval_us(const P& p) {
-    return 0.0033 * eval_work(p, D);
+    return 0.0033 * EvalWork<P>::of(p, D);
 }
 
 /* k_grow's time for the splits of an integral of n regions, us: a step for each 256, which
