@@ -122,3 +122,59 @@ def test_no_handover_by_size_alone(fresh, monkeypatch, n, deepen):
     for b in bufs:
         b.free()
     assert fresh.last_generation()["handovers"] == 0
+
+
+def test_more_room_in_the_tree(fresh, monkeypatch):
+    """A constant in 3 dims: 100 regions take 1023 nodes, more than 8 a region and 64.  The
+    rounds find the room, the class keeps it, and the workgroup has it from then on."""
+    f, integ = I.poly([(0.7, (0, 0, 0))], 3), V.Integrator(99, 2, 5)
+    ways, outs = [], []
+    for k in range(4):
+        if k == 3:
+            monkeypatch.setenv("VMX_DEFER", "0")
+        outs.append((_bins(fresh, f, integ, (7, 5)), fresh.export_regions(3)))
+        g = fresh.last_generation()
+        ways.append((g["workgroup_steps"] > 0, g["rounds"] > 0, g["handovers"]))
+    assert ways == [(True, True, 1), (False, True, 0), (True, False, 0), (False, True, 0)]
+    for b, r in outs[1:]:
+        assert np.array_equal(b, outs[0][0])
+        for key, v in r.items():
+            assert np.array_equal(v, outs[0][1][key]), key
+
+
+# one integral that starts in a workgroup and goes on in the deferred rounds (65536 regions
+# and more), with the candidates' counts and the histogram that the workgroup left
+@pytest.mark.parametrize("f,res,dt", [(POLY2, (24, 20), np.float32), (POLY2, (24, 20), np.float64),
+                                      (I.config4_integrand(3), (40, 30), np.float32),
+                                      (I.moving_blobs(3, 6), (16, 12), np.float32),
+                                      (I.poly([(1.0, (3,)), (0.5, (1,))], 1, step=([1.0], 0.37, 0.25)), (40,), np.float32)],
+                         ids=["poly2", "poly2_f64", "blobs2", "moving3", "poly1"])
+def test_goes_on_in_deferred_rounds(fresh, monkeypatch, f, res, dt):
+    integ = V.Integrator(69999, 1, 5)
+    got = _bins(fresh, f, integ, res, dt), fresh.export_regions(f.dim)
+    g = fresh.last_generation()
+    assert g["workgroup_steps"] > 0 and g["rounds"] > 0 and g["handovers"] == 0
+    monkeypatch.setenv("VMX_DEFER", "0")
+    want = _bins(fresh, f, integ, res, dt), fresh.export_regions(f.dim)
+    assert fresh.last_generation()["workgroup_steps"] == 0
+    assert np.array_equal(got[0], want[0])
+    for key, v in want[1].items():
+        assert np.array_equal(v, got[1][key]), key
+
+
+@pytest.mark.parametrize("n", [6145, 8192, 20000, 70000])
+@pytest.mark.parametrize("f,res", [(I.config4_integrand(3), (32, 20)), (I.poly([(1.0, (3,)), (0.5, (1,))], 1), (32,))],
+                         ids=["blobs2", "poly1"])
+def test_goes_on_in_learned_rounds(fresh, monkeypatch, f, res, n):
+    p = (np.random.default_rng(5).standard_normal(V.refiner_size(f.dim)[0]) * 0.1).astype(np.float32)
+    p[-2], p[-1] = -20.0, 4.0  # mu, sigma
+    fresh.refiner_set(f.dim, p)
+    integ = V.Integrator(n - 1, 1, 5, refiner=V.REFINER_LEARNED)
+    got = _bins(fresh, f, integ, res), fresh.export_regions(f.dim)
+    g = fresh.last_generation()
+    assert g["workgroup_steps"] > 0 and g["rounds"] > 0 and g["handovers"] == 0
+    monkeypatch.setenv("VMX_DEFER", "0")
+    want = _bins(fresh, f, integ, res), fresh.export_regions(f.dim)
+    assert np.array_equal(got[0], want[0])
+    for key, v in want[1].items():
+        assert np.array_equal(v, got[1][key]), key
