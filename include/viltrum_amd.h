@@ -167,8 +167,8 @@ typedef struct vmx_stats {
     uint64_t evals_regions;    /* integrand evaluations for region nodes */
     uint64_t evals_residual;   /* integrand evaluations for the residual */
     uint64_t ties_unresolved;  /* boundary ties broken by geometric order (canonical only) */
-    /* host clock between the phases' readbacks; small integrals end generation without one,
-       so their ms_generate is the time to launch it and ms_stratify holds its device time */
+    /* host clock between the phases' readbacks; the generation of small integrals, which
+       ends without one, by the device's clock */
     double ms_generate, ms_select, ms_stratify, ms_bins, ms_total;
 } vmx_stats;
 

@@ -85,3 +85,21 @@ def test_series_over_an_infinite_range(ctx, rd, decay, mc, n, workgroup):
     it = V.integrator_crespo2021_infinite(rd, n - 1, mc, 2, seed=3)
     V.integrate(it, np.zeros((9, 8, 7)[:rd], dtype=np.float32), I.dyson(decay), V.range_primary_infinite(), ctx=ctx)
     assert (ctx.last_generation()["rounds"] == 0) == workgroup
+
+
+def test_generation_time_of_small_integrals(ctx):
+    """8 times the regions take several times the steps: the time is the generation's, not its
+    launch's, and the phases do not count it twice."""
+    ms = {}
+    for n in (700, 6000):
+        it = V.Integrator(n - 1, 2, 3)
+        best = 1e9
+        for _ in range(8):
+            b = np.zeros((24, 17), dtype=np.float32)
+            V.integrate(it, b, BLOBS, V.range_primary(2), ctx=ctx)
+            s = it.last_stats
+            assert ctx.last_generation()["rounds"] == 0
+            assert s.ms_generate + s.ms_select + s.ms_stratify <= s.ms_total and s.ms_stratify >= 0
+            best = min(best, s.ms_generate)
+        ms[n] = best
+    assert ms[6000] > 1.5 * ms[700] > 0.05, ms

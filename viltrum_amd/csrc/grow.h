@@ -765,6 +765,7 @@ __global__ void __launch_bounds__(GROW_THREADS)
     const Job<T>& jb = g.jobs[j];
     const F& f = fs[j];
     const TreeArrays<T> t = g.t;
+    const uint64_t start = wall_clock64();
     const uint32_t base = jb.node_base, need = jb.N - 1;
     const uint32_t cap = jb.node_cap < GROW_MAX_NODES ? jb.node_cap : GROW_MAX_NODES;
     const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6;
@@ -1045,6 +1046,7 @@ __global__ void __launch_bounds__(GROW_THREADS)
             rt.ties = L.ties;
             if (n == NONE && done && count < need) n = 0;  // too few nodes exist: no route gives N regions
             if (n == NONE) rt.flags |= JF_HANDOVER;
+            atomicMax(g.rounds + 6, uint32_t(wall_clock64() - start));
         }
         return;
     }

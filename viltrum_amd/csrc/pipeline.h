@@ -435,7 +435,7 @@ struct GenArgs {
     uint32_t* cstart;  // [2*J] first slot of the round's candidates (they are contiguous)
     uint32_t* ncand;   // [2*J] number of candidates
     T* theta;         // [J]
-    uint32_t* rounds; // [0] rounds that had candidates, [1] steps of k_grow
+    uint32_t* rounds; // [0] rounds that had candidates, [1] steps of k_grow, [6] its longest block's clock ticks
     uint32_t* depth;  // [D] most splits along each dim over all nodes (block maxima)
     uint32_t J;
     uint32_t max_rounds;

@@ -209,9 +209,9 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     uint32_t cap_total = 0;
     std::vector<vmx::JobRt> rt(J);
     // the rounds' shared state, one block so that one copy reads it back: candidate
-    // counts (2 x J), job states (J), 16 words of counters ([0] rounds, [2..5] the pair
-    // totals after stratification, [8 + d] deepest split count along dim d) and deferred
-    // candidate counts (2 x J)
+    // counts (2 x J), job states (J), 16 words of counters ([0] rounds, [1] and [6] k_grow's
+    // steps and clock, [2..5] the pair totals after stratification, [8 + d] deepest split
+    // count along dim d) and deferred candidate counts (2 x J)
     const size_t state_bytes = sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J + 64 + sizeof(uint32_t) * 2 * J;
     const size_t slot_bytes = (state_bytes + 255) & ~size_t(255);
     char* d_state = nullptr;
@@ -477,7 +477,7 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         ctx->round_hint[hint_key] = small_h[0];
         break;
     }
-    const double ms_gen = ms_since(t_start);
+    double ms_gen = ms_since(t_start);
 
     if constexpr (vmx::IsFubini<P>::value || D > LEARN_MAX_DIM) {
         if (pairs_req) throw VmxError(VMX_ERR_UNSUPPORTED, "training pairs: not for the Fubini form or D > 5");
@@ -728,19 +728,22 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     HIP_CHECK(hipGetLastError());
     uint32_t pairs = 0, nfp = 0;
     uint64_t pairs64 = 0;
+    double ms_grow = 0;  // k_grow by the device's clock: its launch returns at once
     {
         char* pin = static_cast<char*>(ensure_pinned(ctx, state_bytes));
         HIP_CHECK(hipMemcpyAsync(pin, d_state, state_bytes, hipMemcpyDeviceToHost, st));
         HIP_CHECK(hipStreamSynchronize(st));
-        uint32_t w[4];
-        std::memcpy(w, pin + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J + 2 * sizeof(uint32_t), sizeof(w));
-        pairs64 = uint64_t(w[0]) | (uint64_t(w[1]) << 32);
-        pairs = w[2];
-        nfp = w[3];
+        uint32_t w[7];
+        std::memcpy(w, pin + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, sizeof(w));
+        pairs64 = uint64_t(w[2]) | (uint64_t(w[3]) << 32);
+        pairs = w[4];
+        nfp = w[5];
         std::memcpy(rt.data(), pin + sizeof(uint32_t) * 2 * J, sizeof(vmx::JobRt) * J);
         if (grow_all) {
-            std::memcpy(w, pin + sizeof(uint32_t) * 2 * J + sizeof(vmx::JobRt) * J, 2 * sizeof(uint32_t));
             grow_steps = w[1];
+            int khz = 0;
+            HIP_CHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+            if (khz > 0) ms_grow = std::min(double(w[6]) / khz * ((J + uint32_t(n_cu) - 1) / uint32_t(n_cu)), ms_since(t_str));
         }
     }
     ctx->generated.rounds += rounds;
@@ -809,7 +812,8 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
         vmx::k_list_prefix<T><<<1024, 256, 0, st>>>(d_off, d_qlong, d_lst, fa, lp);
     }
     HIP_CHECK(hipGetLastError());
-    const double ms_str = ms_since(t_str);
+    ms_gen += ms_grow;
+    const double ms_str = ms_since(t_str) - ms_grow;
 
     // ---------------- 4. bins
     // one lane per bin, one block per tile of 256 bins of one job
