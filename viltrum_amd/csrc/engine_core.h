@@ -328,12 +328,13 @@ double grow_us(bool learn, double n, double eval) {
 }
 /* What the rounds and their selection cost more than k_grow without those steps, us: two
    launches a round, a round per level, more of both with many integrals, and the chip's
-   time for the splits.  Fitted with the steps above to both generators over 2400 calls: polynomials of 1 to 12
-   terms, 1 to 64 static and 2 to 32 moving blobs, Fubini forms, learned priorities, 2 to
-   6144 regions, 1 to 300 integrals.  Where this rule takes k_grow it is at most 4 % behind
-   the rounds, but for two of those calls (7 %); where it takes the rounds they are at most
-   30 % behind, beside the line.  FP64 in 3 dims spills (a child is 27 values in a lane):
-   rounds from 100 to 300 regions on, one integral. */
+   time for the splits.  Fitted with the steps above to both generators over 2500 calls:
+   polynomials of 1 to 12 terms, 1 to 64 static and 2 to 32 moving blobs, Fubini forms,
+   learned priorities, 2 to 6144 regions, 1 to 300 integrals.  Where this rule takes k_grow
+   it is at most 4 % behind the rounds, but for two of those calls (7 %); where it takes the
+   rounds they are at most 30 % behind, beside the line (38 % in 1 dim with 32 samples a
+   node).  FP64 in 3 dims spills (a child is 27 values in a lane): rounds from 100 to 300
+   regions on, one integral. */
 template <typename T, int D>
 double rounds_us(bool learn, double n, double jobs, double splits) {
     const double base = learn ? 30.0 : (D == 3 && sizeof(T) == 8 ? 30.0 : 40.0);

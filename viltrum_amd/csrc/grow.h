@@ -24,7 +24,8 @@
  * kernels.h for why any order of expansion selects the same N - 1 nodes.
  *
  * A job whose pool reaches Job::grow_stop hands over: its nodes so far become the first
- * candidates of the round kernels.
+ * candidates of the round kernels.  One that is meant to end here and cannot (pool or tree
+ * full, a split too deep) says so, and the rounds generate its batch from the start.
  */
 #ifndef VMX_GROW_H
 #define VMX_GROW_H

@@ -2106,7 +2106,8 @@ inline uint32_t rm_tiles(int db, const uint64_t* res, uint64_t nbins) {
    dims share regions, so far more waves hold bins of one region each than with runs of a
    row (an edge of small regions crosses every row, but few squares).  Narrow grids keep
    runs of 256 bins (a square would stick out), and so does FP64, which has no loop for
-   single regions (301 x 217 bins of 20000 regions, 64 spp: 190 us in runs, 215 us in squares).  FP32, 64 integrals of 512 x 512 bins and 4096 regions, 16 spp: the
+   single regions (301 x 217 bins of 20000 regions, 64 spp: 190 us in runs, 215 us in
+   squares).  FP32, 64 integrals of 512 x 512 bins and 4096 regions, 16 spp: the
    single-region loop in runs 1418 us, in squares 1232 us. */
 template <typename T>
 inline bool bins_tiled(int db, const uint64_t* res) {

@@ -3,8 +3,10 @@
  *
  * Pipeline of a batch of integrals of one (scalar, D, family) (run_batch; one
  * integral is a batch of one):
- *   1. k_roots, then per refinement round k_theta_round + k_expand_round (launched in
- *      chunks; the host checks for remaining candidates between chunks).
+ *   1. small integrals: k_grow, which selects and orders the regions too.  Else k_roots (a
+ *      larger one alone: k_grow's first steps), then per refinement round k_theta_round +
+ *      k_expand_round (launched in chunks; the host checks for remaining candidates between
+ *      chunks).
  *   2. exact selection of the N-1 split nodes per integral on the device (canonical
  *      order), or, for the reference's heap-array order, libstdc++ push_heap/pop_heap
  *      replayed on the host over the GPU-computed errors
@@ -13,8 +15,8 @@
  *      footprints, per-bin footprint lists (pairs emitted per footprint at scanned
  *      offsets, stable radix sort by bin, boundary offsets).
  *   4. k_bins1: per-bin control variate + residual Monte Carlo, one lane per bin.
- * Host synchronisation: after generation (capacity check) and once to size the bin
- * lists.
+ * Host synchronisation: after generation by rounds (capacity check; k_grow's flags come
+ * with the totals) and once to size the bin lists.
  */
 #ifndef VMX_RUN_BATCH_H
 #define VMX_RUN_BATCH_H
@@ -164,13 +166,14 @@ int run_batch(vmx_ctx* ctx, const std::vector<JobIn>& in, hipStream_t st, PairsR
     hint_key[6] = uint64_t(ilog2(n_max));
     // One workgroup per integral generates it (grow.h) where that beats the rounds, both
     // sides as measured (engine_core.h): a 2-D integral of 1024 / 2048 / 4096 regions takes
-    // 370 / 400 / 500 us by rounds, 80 / 115 / 230 here; 64 learned ones of 4096 regions
-    // 1520 -> 430; 3 dims with 8 blobs cross over near 2500 regions.  A larger integral
-    // alone starts here (the rounds of a handful of regions are all launch) and hands over
-    // once its pool fills the chip's first workgroups: 3 to 25 % of a call in 1 dim and in 2
-    // (nothing there from 15 us an evaluation, a loss from 20), 1 to 6 % in 3 from 400
-    // regions (nothing at 2 us, a loss above; FP64 loses 8 to 30 %).  The reference's order replays a heap over the rounds' nodes.
-    // VMX_DEFER chooses among forms of the rounds, so every call with it set runs them.
+    // 255 / 326 / 400 us by rounds and selection, 114 / 172 / 221 here, 64 of 4096 regions
+    // 927 -> 299, 64 learned ones 1189 -> 580; 3 dims with 8 blobs cross over near 2400
+    // regions.  A larger integral alone starts here (the rounds of a handful of regions are
+    // all launch) and hands over once its pool fills the chip's first workgroups: 3 to 25 %
+    // of a call in 1 dim and in 2 (nothing there from 15 us an evaluation, a loss from 20),
+    // 1 to 6 % in 3 from 400 regions (nothing at 2 us, a loss above; FP64 loses 8 to 30 %).
+    // The reference's order replays a heap over the rounds' nodes.  VMX_DEFER chooses among
+    // forms of the rounds, so every call with it set runs them.
     bool grow_all = grow_built<D>(learn) && !replay && !pairs_req && !left && !std::getenv("VMX_DEFER");
     bool grow_start = grow_all && J == 1 && (D <= 2 || sizeof(T) == 4);
     if (grow_all) {
